@@ -215,6 +215,19 @@ int64_t head_argmax_part_floats(int64_t m, int64_t n);
 int launch_head_argmax(const float* x, int64_t m, int64_t k, const float* w, int64_t ldb,
                        int64_t n, const float* bias, float* part, float* pairs, hipStream_t s);
 
+// The same over a weight packed once as float16 pairs (qph_head.hip): K = 256,
+// closer to float64 than the float32 chain.  head_split_pack leaves wp NULL
+// for a weight or bias that cannot be split (infinities, NaN, past 2^60).
+struct HeadSplit {
+  char* wp = nullptr;         // owned by the caller (hipFree)
+  const float* ci = nullptr;  // inside wp's allocation
+};
+bool head_split_eligible(int64_t k, int64_t n);
+int64_t head_split_scratch_floats(int64_t m, int64_t n);   // for every row count up to m
+int head_split_pack(const float* w, int64_t n, const float* bias, HeadSplit* out, hipStream_t s);
+int launch_head_split(const float* x, int64_t m, const HeadSplit& hs, const float* w, int64_t n,
+                      const float* bias, float* scratch, float* pairs, hipStream_t s);
+
 // The session's linears: C[M][N] = act(A[M][K] * Wt[N][K]^T + bias) (+ res),
 // Wt the weight held transposed (k contiguous).
 struct LinArgs {

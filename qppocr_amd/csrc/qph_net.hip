@@ -39,6 +39,7 @@ struct qph_net {
   std::vector<bool> head;        // linear node i and the pairs-only softmax i + 1 run fused
   std::vector<bool> qa_fused;    // linear node i (QKV) and attention node i + 1, one launch
   std::vector<float*> head_part; // per fused head: its per-block argmax partials
+  std::vector<HeadSplit> head_split; // per fused head: its packed weight (wp NULL: unsplit kernels)
   std::vector<bool> nostore;     // per tensor: never materialised (inside one fused launch)
   std::vector<float*> tptr;      // per tensor device pointer
   std::vector<int64_t> pitch;    // per tensor: padded row pitch in floats (0: contiguous)
@@ -242,6 +243,7 @@ static void plan_fused_head(qph_net* net, int32_t flags) {
   const size_t nn = net->nodes.size(), nt = net->tptr.size();
   net->head.assign(nn, false);
   net->head_part.assign(nn, nullptr);
+  net->head_split.assign(nn, HeadSplit{});
   net->nostore.assign(nt, false);
   if (!(flags & QPH_NET_FUSED_HEAD)) return;
   auto ok = [&](int32_t t) { return t >= 0 && (size_t)t < nt; };
@@ -953,11 +955,15 @@ static int run_all(qph_net* net) {
       const qph_node& q = net->nodes[i];
       const qph_node& r = net->nodes[i + 1];
       const int64_t k = q.ws[0], nn = q.ws[1];
+      const float* bias = q.bias >= 0 ? net->weights[q.bias] : nullptr;
+      const int64_t rows = numel_of(net, q.in) / k;
       const float* w = net->wk[i] ? net->wk[i] : net->weights[q.w];
       const int64_t ldb = net->wk[i] ? (nn + 3) / 4 * 4 : nn;
-      const int rc = launch_head_argmax(net->tptr[q.in], numel_of(net, q.in) / k, k, w, ldb, nn,
-                                        q.bias >= 0 ? net->weights[q.bias] : nullptr,
-                                        net->head_part[i], net->tptr[r.out2], s);
+      const int rc = net->head_split[i].wp
+                         ? launch_head_split(net->tptr[q.in], rows, net->head_split[i], w, nn, bias,
+                                             net->head_part[i], net->tptr[r.out2], s)
+                         : launch_head_argmax(net->tptr[q.in], rows, k, w, ldb, nn, bias,
+                                              net->head_part[i], net->tptr[r.out2], s);
       if (rc != QPH_OK) return fail(rc, node_name(i, q) + ": " + qph_last_error());
       step = 2;
     } else if (net->fpn[i]) {
@@ -1077,6 +1083,8 @@ static void release(qph_net* net) {
     if (p) (void)hipFree(p);
   for (float* p : net->head_part)
     if (p) (void)hipFree(p);
+  for (HeadSplit& h : net->head_split)
+    if (h.wp) (void)hipFree(h.wp);
   for (float* p : net->fpn_tmp)
     if (p) (void)hipFree(p);
   for (float* p : net->wt)
@@ -1210,6 +1218,12 @@ QPH_API int qph_net_create(qph_ctx* ctx, const qph_net_spec* spec,
                                      ctx->stream, n.cp.group);
       if (rc) return bail(rc);
     }
+    if (net->head[i] && head_split_eligible(n.ws[0], n.ws[1])) {
+      rc = head_split_pack(net->weights[n.w], n.ws[1], n.bias >= 0 ? net->weights[n.bias] : nullptr,
+                           &net->head_split[i], ctx->stream);
+      if (rc) return bail(rc);
+      if (net->head_split[i].wp) continue;
+    }
     if (n.op == QPH_OP_LINEAR) {
       // below the 128x128 size: weight kept transposed for linear_nt_kernel
       const int64_t k = n.ws[0], nn = n.ws[1], rows = numel_of(net, n.in) / k;
@@ -1246,8 +1260,9 @@ QPH_API int qph_net_create(qph_ctx* ctx, const qph_net_spec* spec,
     const qph_node& q = net->nodes[i];
     const int64_t rows = numel_of(net, q.in) / q.ws[0];
     float* d = nullptr;
-    rc = hip_check(hipMalloc((void**)&d, (size_t)head_argmax_part_floats(rows, q.ws[1]) * 4),
-                   "hipMalloc(head partials)");
+    const int64_t floats = net->head_split[i].wp ? head_split_scratch_floats(rows, q.ws[1])
+                                                 : head_argmax_part_floats(rows, q.ws[1]);
+    rc = hip_check(hipMalloc((void**)&d, (size_t)floats * 4), "hipMalloc(head partials)");
     if (rc) return bail(rc);
     net->head_part[i] = d;
   }
@@ -1331,7 +1346,7 @@ QPH_API int qph_net_plan(qph_net* net, int32_t* first, int32_t* nodes, int32_t* 
     size_t step = 1;
     int32_t nk = 1;
     if (net->group_len[i] > 1) step = (size_t)net->group_len[i];
-    else if (net->head[i]) step = 2, nk = 2;
+    else if (net->head[i]) step = 2, nk = net->head_split[i].wp ? 3 : 2;
     else if (net->fused[i]) step = net->dwpw[i].stem ? 3 : 2;
     else if (net->convt_fused[i]) step = 2;
     else if (net->qa_fused[i]) step = 2;
