@@ -961,187 +961,202 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
   }
 }
 
-// Head dimension known at compile time: one workgroup per (batch, head);
-// q (times scale: the Mul node), k and v of all T rows arrive in LDS in one
-// burst of loads, then the query rows go in blocks (all rows up to 64).
-// Scores: one chain of DH fmas per (row, key).  Softmax: eight threads per
-// row, thread j owning elements j, j+8, ... -- its max part, its exp1 values
-// and exactly the reference's lane-j chain -- then the
+// Head dimension known at compile time: a workgroup owns a block of query rows
+// of one (batch, head), eight threads a row.  Both products run on
+// v_mfma_f32_16x16x4f32, whose four k terms per instruction are added in
+// order, so each 16x16 output block is the reference's fma chains (k = d for
+// the scores, k = j for P.V, each from +0).  Softmax: thread j of a row owns
+// elements j, j+8, ... in registers -- its max part, its exp1 values and
+// exactly the reference's lane-j chain -- then the
 // ((l0+l4)+(l1+l5))+((l2+l6)+(l3+l7)) tree and the tail in order within the
-// group of eight (no workgroup barrier).  P.V: one chain of T fmas per
-// (row, d).
-// MF (T % 4 == 0): both products on v_mfma_f32_16x16x4f32, whose four k
-// terms per instruction are added in order, so each 16x16 output block is
-// the same fma chains (k = d for the scores, k = j for P.V, each from 0);
-// q, k and v rows are zero-filled up to a multiple of 16 and the score /
-// probability block to 16-row, 16-column tiles, whose extra outputs are
-// never used.
+// group of eight (no workgroup barrier).
+// Rows and columns past t are padding: q, k and v rows up to a multiple of 16
+// are zero, and the probabilities of columns t .. up to a multiple of 4 are
+// written as zeros, whose terms 0 * 0 leave a chain's value as it is (a chain
+// from +0 is never -0).  Outputs of padding rows and columns are never used.
+// LDS rows are DH + 4 words (q, k, v) and tp + 4 (probabilities), so the 16
+// rows x 4 terms of an operand read fall on 64 banks.
 
-// The attention of one (batch, head) once q (times scale), k and v of its
-// rows are in LDS (rows t .. tp - 1 zero): scores, the softmax with the
-// reference's lane chains, P.V, written to out[r * D + d] (out at the
-// head's first column of the batch's first row).  NT threads.
-template <int DH, bool MF, int NT>
-__device__ __forceinline__ void attention_rows(const float* sq, const float* sk, const float* sv,
-                                               float* sp, int t, int tp, int ldp, int blk,
-                                               int64_t D, float* __restrict__ out) {
-  constexpr int LD = DH + 1;
-  const int full = t >= 8 ? (t / 8) * 8 : 0;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// The block's rb rows once q (times scale, the block's rows), k and v are in
+// LDS; out at the head's first column of the block's first row, rows D apart.
+// blockDim.x >= 8 rb; NE >= t / 8 elements a thread.
+template <int DH, int NE>
+__device__ __forceinline__ void attention_block(const float* sq, const float* sk, const float* sv,
+                                                float* sp, int rb, int t, int tp, int64_t D,
+                                                float* __restrict__ out) {
+  constexpr int LD = DH + 4;
+  const int ldp = tp + 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
   const int lg = lane >> 4, l16 = lane & 15;
-  for (int r0 = 0; r0 < t; r0 += blk) {
-    const int rb = (t - r0) < blk ? (t - r0) : blk;
-    if (MF) {
-      // S block (rb x t) in 16x16 tiles over the waves
-      const int nr = (rb + 15) / 16, nc = tp / 16;
-      for (int tl = wave; tl < nr * nc; tl += NT / 64) {
-        const int br = tl / nc, bc = tl - br * nc;
-        const float* a = sq + (r0 + 16 * br + l16) * LD + lg;
-        const float* bk = sk + (16 * bc + l16) * LD + lg;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  const int nr = (rb + 15) / 16, nc = tp / 16;
+  // S block (rb x t) in 16x16 tiles over the waves
+  // (one key tile and two query tiles at a time: two chains)
+  const int np = (nr + 1) / 2;
+  for (int tl = wave; tl < np * nc; tl += nw) {
+    const int bp = tl / nc, bc = tl - bp * nc;
+    const int br0 = 2 * bp, br1 = min(2 * bp + 1, nr - 1);
+    const float* a0 = sq + (16 * br0 + l16) * LD + lg;
+    const float* a1 = sq + (16 * br1 + l16) * LD + lg;
+    const float* bk = sk + (16 * bc + l16) * LD + lg;
+    f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
 #pragma unroll
-        for (int s4 = 0; s4 < DH / 4; s4++)
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[4 * s4], bk[4 * s4], acc, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 4; v++) sp[(16 * br + 4 * lg + v) * ldp + 16 * bc + l16] = acc[v];
-      }
-    } else {
-      // scores S[r][j] = chain over d of fma(q[r][d], k[j][d], acc)
-      for (int i = tid; i < rb * t; i += NT) {
-        const int r = i / t, j = i - r * t;
-        const float* qr = sq + (r0 + r) * LD;
-        const float* kj = sk + j * LD;
-        float acc = 0.0f;
-#pragma unroll
-        for (int d = 0; d < DH; d++) acc = __builtin_fmaf(qr[d], kj[d], acc);
-        sp[r * ldp + j] = acc;
-      }
-    }
-    __syncthreads();
-    // softmax, eight threads per row (groups never straddle a wave)
-    for (int g0 = 0; g0 < rb; g0 += NT / 8) {
-      const int r = g0 + (tid >> 3), lj = tid & 7;
-      const bool rowok = r < rb;
-      float* pr = sp + (rowok ? r : 0) * ldp;
-      float mx = -__builtin_inff();
-      if (rowok)
-        for (int j = lj; j < t; j += 8) mx = fmaxf(mx, pr[j]);
-      for (int off = 4; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 8));
-      if (t < 8 && rowok) {   // narrow rows: sequential max from the first element
-        mx = pr[0];
-        for (int j = 1; j < t; j++)
-          if (pr[j] > mx) mx = pr[j];
-      }
-      float s = 0.0f;
-      if (rowok)
-        for (int j = lj; j < t; j += 8) {
-          const float e = exp1(pr[j] - mx);
-          pr[j] = e;
-          if (j < full) s = s + e;   // lane lj's chain, ascending j
-        }
-      // tree of the eight lane chains, then the tail in order (lane 0)
-      const int gb = (threadIdx.x & 63) & ~7;
-      const float l0 = __shfl(s, gb + 0, 64), l1 = __shfl(s, gb + 1, 64);
-      const float l2 = __shfl(s, gb + 2, 64), l3 = __shfl(s, gb + 3, 64);
-      const float l4 = __shfl(s, gb + 4, 64), l5 = __shfl(s, gb + 5, 64);
-      const float l6 = __shfl(s, gb + 6, 64), l7 = __shfl(s, gb + 7, 64);
-      float sum = 0.0f;
-      if (rowok && lj == 0) {
-        if (t >= 8) sum = ((l0 + l4) + (l1 + l5)) + ((l2 + l6) + (l3 + l7));
-        for (int j = full; j < t; j++) sum = sum + pr[j];
-      }
-      sum = __shfl(sum, gb, 64);
-      const float inv = 1.0f / sum;
-      if (rowok)
-        for (int j = lj; j < t; j += 8) pr[j] = pr[j] * inv;
-    }
-    __syncthreads();
-    if (MF) {
-      // O block (rb x DH) = P . v in 16x16 tiles, k = j over exactly t terms
-      const int nr = (rb + 15) / 16;
-      for (int tl = wave; tl < nr * (DH / 16); tl += NT / 64) {
-        const int br = tl / (DH / 16), bc = tl - br * (DH / 16);
-        const float* a = sp + (16 * br + l16) * ldp + lg;
-        const float* bv = sv + lg * LD + 16 * bc + l16;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s4 = 0; s4 < t / 4; s4++)
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[4 * s4], bv[4 * s4 * LD], acc, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int r = 16 * br + 4 * lg + v;
-          if (r < rb) out[(int64_t)(r0 + r) * D + 16 * bc + l16] = acc[v];
-        }
-      }
-    } else {
-      // O[r][d] = chain over j of fma(P[r][j], v[j][d], acc); operands read
-      // eight j at a time so their LDS reads are in flight together
-      for (int i = tid; i < rb * DH; i += NT) {
-        const int r = i / DH, d = i - r * DH;
-        const float* p = sp + r * ldp;
-        const float* vd = sv + d;
-        float acc = 0.0f;
-        int j = 0;
-        for (; j + 8 <= t; j += 8) {
-          float pv[8], vv[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) {
-            pv[u] = p[j + u];
-            vv[u] = vd[(j + u) * LD];
-          }
-#pragma unroll
-          for (int u = 0; u < 8; u++) acc = __builtin_fmaf(pv[u], vv[u], acc);
-        }
-        for (; j < t; j++) acc = __builtin_fmaf(p[j], vd[j * LD], acc);
-        out[(int64_t)(r0 + r) * D + d] = acc;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-template <int DH, bool MF>
-__global__ __launch_bounds__(256) void attention_dh_kernel(const float* __restrict__ qkv,
-                                                           int64_t T, int64_t H, float scale,
-                                                           int blk, float* __restrict__ out) {
-  extern __shared__ float sm[];
-  constexpr int LD = DH + 1;
-  const int64_t b = blockIdx.x / H, h = blockIdx.x - b * H;
-  const int tid = threadIdx.x;
-  const int64_t D = H * DH;
-  const int t = (int)T;
-  const int tp = MF ? (t + 15) / 16 * 16 : t;     // rows held (zero past t)
-  const int ldp = MF ? tp + 1 : t + 1;
-  float* sq = sm;                 // tp x LD (scaled q)
-  float* sk = sq + tp * LD;       // tp x LD
-  float* sv = sk + tp * LD;       // tp x LD
-  float* sp = sv + tp * LD;       // blk (rounded to 16) x ldp scores / probabilities
-  const float* base = qkv + b * T * 3 * D + h * DH;
-  for (int i0 = tid; i0 < tp * DH; i0 += 256 * 4) {
-    float q[4], k[4], v[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int i = i0 + 256 * u;
-      q[u] = k[u] = v[u] = 0.0f;
-      if (i < t * DH) {
-        const float* row = base + (int64_t)(i / DH) * 3 * D + (i % DH);
-        q[u] = row[0];
-        k[u] = row[D];
-        v[u] = row[2 * D];
-      }
+    for (int s4 = 0; s4 < DH / 4; s4++) {
+      const float k = bk[4 * s4];
+      acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[4 * s4], k, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[4 * s4], k, acc1, 0, 0, 0);
     }
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int i = i0 + 256 * u;
-      if (i < tp * DH) {
-        const int r = i / DH, d = i - r * DH;
-        sq[r * LD + d] = q[u] * scale;   // Mul node
-        sk[r * LD + d] = k[u];
-        sv[r * LD + d] = v[u];
-      }
+    for (int v = 0; v < 4; v++) {
+      sp[(16 * br0 + 4 * lg + v) * ldp + 16 * bc + l16] = acc0[v];
+      sp[(16 * br1 + 4 * lg + v) * ldp + 16 * bc + l16] = acc1[v];
     }
   }
   __syncthreads();
-  attention_rows<DH, MF, 256>(sq, sk, sv, sp, t, tp, ldp, blk, D, out + b * T * D + h * DH);
+  const int r = tid >> 3, lj = tid & 7;
+  if (r < 16 * nr) {   // groups of eight are whole
+    const int full = t >= 8 ? (t / 8) * 8 : 0;
+    float* pr = sp + r * ldp;
+    float e[NE];
+    float mx = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      if (8 * i >= t) break;   // (uniform)
+      e[i] = lj + 8 * i < t ? pr[lj + 8 * i] : -__builtin_inff();
+      mx = fmaxf(mx, e[i]);
+    }
+#pragma unroll
+    for (int off = 4; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 8));
+    if (t < 8) {   // narrow rows: sequential max from the first element
+      mx = __shfl(e[0], 0, 8);
+      for (int j = 1; j < t; j++) {
+        const float o = __shfl(e[0], j, 8);
+        if (o > mx) mx = o;
+      }
+    }
+    float s = 0.0f, last = 0.0f;   // the lane's chain, its element past the whole eights
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      if (8 * i >= t) break;
+      e[i] = exp1(e[i] - mx);
+      if (8 * i < full) s = s + e[i];
+      else last = e[i];   // (past t: of -inf, never added)
+    }
+    const float l0 = __shfl(s, 0, 8), l1 = __shfl(s, 1, 8), l2 = __shfl(s, 2, 8);
+    const float l3 = __shfl(s, 3, 8), l4 = __shfl(s, 4, 8), l5 = __shfl(s, 5, 8);
+    const float l6 = __shfl(s, 6, 8), l7 = __shfl(s, 7, 8);
+    float sum = t >= 8 ? ((l0 + l4) + (l1 + l5)) + ((l2 + l6) + (l3 + l7)) : 0.0f;
+#pragma unroll
+    for (int u = 0; u < 7; u++) {
+      const float o = __shfl(last, u, 8);
+      if (u < t - full) sum = sum + o;
+    }
+    const float inv = 1.0f / sum;
+    const int t4 = (t + 3) / 4 * 4;
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      if (8 * i >= t) break;
+      if (lj + 8 * i < t) pr[lj + 8 * i] = e[i] * inv;
+    }
+    if (lj < t4 - t) pr[t + lj] = 0.0f;
+  }
+  __syncthreads();
+  // O block (rb x DH) = P . v in 16x16 tiles, k = j
+  const int ns = (t + 3) / 4;
+  for (int tl = wave; tl < nr * (DH / 16); tl += nw) {
+    const int br = tl / (DH / 16), bc = tl - br * (DH / 16);
+    const float* a = sp + (16 * br + l16) * ldp + lg;
+    const float* bv = sv + lg * LD + 16 * bc + l16;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    int s4 = 0;
+    for (; s4 + 8 <= ns; s4 += 8) {   // eight steps' operands in flight
+      float pa[8], va[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        pa[u] = a[4 * (s4 + u)];
+        va[u] = bv[4 * (s4 + u) * LD];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[u], va[u], acc, 0, 0, 0);
+    }
+    for (; s4 < ns; s4++)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[4 * s4], bv[4 * s4 * LD], acc, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int i = 16 * br + 4 * lg + v;
+      if (i < rb) out[(int64_t)i * D + 16 * bc + l16] = acc[v];
+    }
+  }
+}
+
+// Attention over stored qkv rows: workgroup (batch and head, block of blk query
+// rows).  Every block loads all k and v rows (from L2 after the first).  One
+// workgroup per (batch, head) that walked its blocks one after another took
+// 70 us at 50 lines x 136 rows x 8 heads (35 now), and 24 us at 19 x 61 (7.9),
+// whose products ran on the vector unit for want of a multiple of 4.  What
+// bounds it now: the softmax's vector instructions (41% of the cycles at 50 x
+// 136, the MFMAs 24%) and the barriers between its phases.
+template <int DH, int NE>
+__global__ __launch_bounds__(512) void attention_dh_kernel(const float* __restrict__ qkv, int t,
+                                                           int H, float scale, int blk, int wide,
+                                                           float* __restrict__ out) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  constexpr int LD = DH + 4, C4 = DH / 4;
+  const int b = blockIdx.x / H, h = blockIdx.x - b * H;
+  const int r0 = blockIdx.y * blk, rb = min(blk, t - r0);
+  const int64_t D = (int64_t)H * DH;
+  const int tp = (t + 15) / 16 * 16, qp = (rb + 15) / 16 * 16;
+  float* sk = sm;                 // tp x LD
+  float* sv = sk + tp * LD;       // tp x LD
+  float* sq = sv + tp * LD;       // blk x LD (scaled q)
+  float* sp = sq + blk * LD;      // blk x (tp + 4) scores / probabilities
+  const float* base = qkv + (int64_t)b * t * 3 * D + h * DH;
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  // rows of four-word chunks (one load each where qkv is 16-byte aligned): k,
+  // v, then the block's q
+  auto load4 = [&](const float* p) {
+    if (wide) return *(const f32x4*)p;
+    const f32x4 w = {p[0], p[1], p[2], p[3]};
+    return w;
+  };
+  // (the loads of a round -- q, and up to four chunks of k and v a thread --
+  // all go out before the first is waited for)
+  const int nt = blockDim.x;
+  f32x4 q[2];
+#pragma unroll
+  for (int u = 0; u < DH / 32; u++) {   // qp C4 <= 8 blk DH / 32
+    const int i = threadIdx.x + u * nt, r = i / C4, c = 4 * (i - r * C4);
+    q[u] = load4(base + (int64_t)min(r0 + r, t - 1) * 3 * D + c);
+  }
+  for (int i0 = threadIdx.x; i0 < tp * C4; i0 += 4 * nt) {
+    f32x4 k[4], v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int i = i0 + u * nt, r = i / C4, c = 4 * (i - r * C4);
+      if (i < tp * C4) {
+        const float* row = base + (int64_t)min(r, t - 1) * 3 * D + c;
+        k[u] = load4(row + D);
+        v[u] = load4(row + 2 * D);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int i = i0 + u * nt, r = i / C4, c = 4 * (i - r * C4);
+      if (i < tp * C4) {
+        *(f32x4*)(sk + r * LD + c) = r < t ? k[u] : zero;
+        *(f32x4*)(sv + r * LD + c) = r < t ? v[u] : zero;
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < DH / 32; u++) {
+    const int i = threadIdx.x + u * nt, r = i / C4, c = 4 * (i - r * C4);
+    const f32x4 y = {q[u][0] * scale, q[u][1] * scale, q[u][2] * scale, q[u][3] * scale};   // Mul
+    if (r < qp) *(f32x4*)(sq + r * LD + c) = r < rb ? y : zero;
+  }
+  __syncthreads();
+  attention_block<DH, NE>(sq, sk, sv, sp, rb, t, tp, D,
+                          out + ((int64_t)b * t + r0) * D + h * DH);
 }
 
 // The rec QKV linear and the attention that reads it, one launch: one
@@ -1164,9 +1179,9 @@ template <int NK>
 __global__ __launch_bounds__(512) void qkv_attention_kernel(const float* __restrict__ x,
                                                             const float* __restrict__ wt,
                                                             const float* __restrict__ bias,
-                                                            int T, int H, float scale, int blk,
+                                                            int T, int H, float scale,
                                                             float* __restrict__ out) {
-  constexpr int DH = 32, LD = DH + 1, K = NK * 64;
+  constexpr int DH = 32, LD = DH + 4, K = NK * 64;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1284,7 +1299,7 @@ __global__ __launch_bounds__(512) void qkv_attention_kernel(const float* __restr
   float* sq = sm;                       // tp x LD (scaled q)
   float* sk = sq + QA_ROWS * LD;        // tp x LD
   float* sv = sk + QA_ROWS * LD;        // tp x LD
-  float* sp = sv + QA_ROWS * LD;        // blk (rounded to 16) x (tp + 1)
+  float* sp = sv + QA_ROWS * LD;        // tp x (tp + 4)
 #pragma unroll
   for (int i = 0; i < 3; i++) {
     const int j = wave + 8 * i, rb = j / 6, cb = j - 6 * rb;
@@ -1300,8 +1315,8 @@ __global__ __launch_bounds__(512) void qkv_attention_kernel(const float* __restr
     }
   }
   __syncthreads();
-  attention_rows<DH, true, 512>(sq, sk, sv, sp, T, tp, tp + 1, blk, D,
-                                out + (int64_t)b * T * D + h * DH);
+  attention_block<DH, QA_ROWS / 8>(sq, sk, sv, sp, T, T, tp, D,
+                                   out + (int64_t)b * T * D + h * DH);
 }
 
 bool qkv_attention_eligible(int64_t batch, int64_t t, int64_t heads, int64_t dh, int64_t k) {
@@ -1319,67 +1334,68 @@ int launch_qkv_attention(const float* x, const float* wt, const float* bias, int
     return fail(QPH_EUNSUPPORTED, "qkv + attention: operands not 16-byte aligned");
   // the two stages (the attention's q, k, v and scores fit in them after)
   const size_t lds = (size_t)2 * QA_STAGE * 4;
-  const int blk = (int)t;   // all query rows in one block
   const dim3 grid((unsigned)(batch * heads));
   switch (k / 64) {
     case 1:
       QPH_TRY(allow_full_lds((const void*)qkv_attention_kernel<1>));
       hipLaunchKernelGGL(qkv_attention_kernel<1>, grid, dim3(512), lds, s, x, wt, bias, (int)t,
-                         (int)heads, scale, blk, out);
+                         (int)heads, scale, out);
       break;
     case 2:
       QPH_TRY(allow_full_lds((const void*)qkv_attention_kernel<2>));
       hipLaunchKernelGGL(qkv_attention_kernel<2>, grid, dim3(512), lds, s, x, wt, bias, (int)t,
-                         (int)heads, scale, blk, out);
+                         (int)heads, scale, out);
       break;
     case 3:
       QPH_TRY(allow_full_lds((const void*)qkv_attention_kernel<3>));
       hipLaunchKernelGGL(qkv_attention_kernel<3>, grid, dim3(512), lds, s, x, wt, bias, (int)t,
-                         (int)heads, scale, blk, out);
+                         (int)heads, scale, out);
       break;
     default:
       QPH_TRY(allow_full_lds((const void*)qkv_attention_kernel<4>));
       hipLaunchKernelGGL(qkv_attention_kernel<4>, grid, dim3(512), lds, s, x, wt, bias, (int)t,
-                         (int)heads, scale, blk, out);
+                         (int)heads, scale, out);
       break;
   }
   return launch_check("qkv_attention_kernel");
 }
 
-static size_t attention_dh_lds(int64_t t, int64_t dh, int64_t blk, bool mf) {
-  const int64_t tp = mf ? (t + 15) / 16 * 16 : t;
-  const int64_t bp = mf ? (blk + 15) / 16 * 16 : blk;
-  return (size_t)(3 * tp * (dh + 1) + bp * (tp + 1)) * sizeof(float);
+static size_t attention_dh_lds(int64_t t, int64_t dh, int64_t blk) {
+  const int64_t tp = (t + 15) / 16 * 16;
+  return (size_t)((2 * tp + blk) * (dh + 4) + blk * (tp + 4)) * sizeof(float);
+}
+
+template <int DH>
+static int launch_attention_dh(const float* qkv, int64_t batch, int64_t t, int64_t heads,
+                               float scale, int64_t blk, float* out, hipStream_t s) {
+  const dim3 grid((unsigned)(batch * heads), ceil_div(t, blk)), block((unsigned)(8 * blk));
+  const size_t lds = attention_dh_lds(t, DH, blk);
+  auto go = [&](auto k) {
+    QPH_TRY(allow_full_lds((const void*)k));
+    hipLaunchKernelGGL(k, grid, block, lds, s, qkv, (int)t, (int)heads, scale, (int)blk,
+                       (int)((uintptr_t)qkv % 16 == 0), out);
+    return launch_check("attention_dh_kernel");
+  };
+  if (t <= 64) return go(attention_dh_kernel<DH, 8>);
+  if (t <= 128) return go(attention_dh_kernel<DH, 16>);
+  if (t <= 256) return go(attention_dh_kernel<DH, 32>);
+  return go(attention_dh_kernel<DH, 40>);
 }
 
 int launch_attention(const float* qkv, int64_t batch, int64_t t, int64_t heads, int64_t dh,
                      float scale, float* out, hipStream_t s) {
-  // query rows per block: all of them up to 64, else 64 or 32 as LDS allows
-  const bool mf = t % 4 == 0;
-  int64_t blk = t <= 64 ? t : 64;
-  if (attention_dh_lds(t, dh, blk, mf) > 160 * 1024) blk = 32;
-  if ((dh == 32 || dh == 64) && attention_dh_lds(t, dh, blk, mf) <= 160 * 1024) {
+  // query rows per block: even blocks of at most 64 (512 threads), fewer
+  // while the launch would leave CUs without a workgroup or LDS is short
+  const int64_t tiles = (t + 15) / 16;
+  int64_t per = (tiles + (tiles + 3) / 4 - 1) / ((tiles + 3) / 4);
+  while (per > 1 && (batch * heads * ((tiles + per - 1) / per) < 256 ||
+                     attention_dh_lds(t, dh, 16 * per) > 160 * 1024))
+    per--;
+  // (the longest rows each head dimension takes; shorter than LDS allows)
+  if ((dh == 32 && t <= 312) || (dh == 64 && t < 180)) {
     if (batch * heads > (1ll << 31)) return fail(QPH_EUNSUPPORTED, "attention: grid too large");
-    const size_t lds = attention_dh_lds(t, dh, blk, mf);
-    const void* fn = dh == 32 ? (mf ? (const void*)attention_dh_kernel<32, true>
-                                    : (const void*)attention_dh_kernel<32, false>)
-                              : (mf ? (const void*)attention_dh_kernel<64, true>
-                                    : (const void*)attention_dh_kernel<64, false>);
-    QPH_TRY(allow_full_lds(fn));
-    const dim3 grid((unsigned)(batch * heads));
-    if (dh == 32 && mf)
-      hipLaunchKernelGGL((attention_dh_kernel<32, true>), grid, dim3(256), lds, s, qkv, t, heads,
-                         scale, (int)blk, out);
-    else if (dh == 32)
-      hipLaunchKernelGGL((attention_dh_kernel<32, false>), grid, dim3(256), lds, s, qkv, t, heads,
-                         scale, (int)blk, out);
-    else if (mf)
-      hipLaunchKernelGGL((attention_dh_kernel<64, true>), grid, dim3(256), lds, s, qkv, t, heads,
-                         scale, (int)blk, out);
-    else
-      hipLaunchKernelGGL((attention_dh_kernel<64, false>), grid, dim3(256), lds, s, qkv, t, heads,
-                         scale, (int)blk, out);
-    return launch_check("attention_dh_kernel");
+    return dh == 32 ? launch_attention_dh<32>(qkv, batch, t, heads, scale, 16 * per, out, s)
+                    : launch_attention_dh<64>(qkv, batch, t, heads, scale, 16 * per, out, s);
   }
   return launch_attention_generic(qkv, batch, t, heads, dh, scale, out, s);
 }
