@@ -1518,12 +1518,16 @@ static void launch_lt(const LinArgs& g, hipStream_t s) {
     hipLaunchKernelGGL((linear_nt_kernel<TM, TN, NS, 0>), grid, dim3(256), 0, s, g, ntiles, per_xcd);
 }
 
-// Tile shape and ring depth as measured on the rec linears (1280 rows, K
-// 256 / 1024, N 256..1024) and 1x1 convs (K 64..256): 32x32 tiles beat 64x32
-// and 64x64 on all of them.  Three stages (48 KB, three workgroups per CU)
-// beat four (two per CU) and, where the slabs are many or the tiles fill
-// three workgroups per CU, two; two stages (32 KB) win for K <= 128 and when
-// the tiles need two rounds at three per CU but one at four (QKV: 960).
+// Tile shape and ring depth as measured on the rec linears (1280 to 6800 rows, K
+// 256 / 1024, N 256..1024) and 1x1 convs (K 64..256).  Up to three 32x32
+// tiles per CU, three stages (48 KB, three workgroups per CU): 1280 x 256 x
+// 1024 14.0 us against 15.5 with two stages and 15.5 with 32x64 tiles.  Past
+// that the tiles come in rounds anyway and two stages (32 KB, five
+// workgroups) hide more: 6800 x 256 x 1024 43.0 -> 39.2 us, 6800 x 256 x 256
+// 16.3 -> 14.4.  From N = 512 on such launches take 32x64 tiles (each x slab
+// read for twice the columns): 6800 x 1024 x 256 59.1 -> 45.8, 6800 x 768 x 256
+// 40.6 -> 31.4, 1280 x 1024 x 256 13.5 -> 12.7 (32x32: 47.8, 34.1, 13.4).
+// 64-row tiles were never the fastest.
 int launch_linear_nt(const LinArgs& g, hipStream_t s) {
   if (!linear_nt_eligible(g.m, g.n, g.k, g.lda))
     return fail(QPH_EUNSUPPORTED, "linear: shape outside the resident-weight kernel");
@@ -1531,10 +1535,12 @@ int launch_linear_nt(const LinArgs& g, hipStream_t s) {
   QPH_TRY(device_cus(nullptr, &cus_i));
   const int64_t tiles = (int64_t)ceil_div(g.m, 32) * ceil_div(g.n, 32);
   const int64_t cus = cus_i;
-  if (g.k <= 128 || (tiles > 3 * cus && tiles <= 4 * cus))
-    launch_lt<32, 32, 2>(g, s);
-  else
+  if (g.k > 128 && tiles <= 3 * cus)
     launch_lt<32, 32, 3>(g, s);
+  else if (g.k > 128 && g.n >= 512)
+    launch_lt<32, 64, 2>(g, s);
+  else
+    launch_lt<32, 32, 2>(g, s);
   return launch_check("linear_nt_kernel");
 }
 
