@@ -912,6 +912,36 @@ static int plan_fpn(qph_net* net) {
   return QPH_OK;
 }
 
+// Nodes the launch that starts at node i covers (the stepping of run_all),
+// without those folded into its epilogue.
+static size_t launch_nodes(const qph_net* net, size_t i) {
+  if (net->group_len[i] > 1) return (size_t)net->group_len[i];
+  if (net->head[i]) return 2;
+  if (net->fused[i]) return net->dwpw[i].stem ? 3 : 2;
+  if (net->convt_fused[i] || net->qa_fused[i]) return 2;
+  return net->fpn[i] ? 4 : 1;
+}
+
+// A 1x1 conv of single-pixel maps ([n, C, 1, 1], after a global pool: the SE
+// gates, the cls net's 1280-wide conv) that has a launch of its own runs as
+// the row-major product over the batch, whose rows x[n][C] and W[M][C] are.
+// As one small GEMM per batch item it took 24 us at 32 x 1280 x 256 (5.7 now).
+// Bias placement: no seeded rows at M % 4 == 0, or all of them (run_node).
+static void plan_single_pixel(qph_net* net) {
+  const size_t nn = net->nodes.size();
+  for (size_t i = 0; i < nn;) {
+    const size_t step = launch_nodes(net, i);
+    const qph_node& q = net->nodes[i];
+    const int64_t* xs = &net->shapes[4 * (size_t)q.in];
+    if (step == 1 && q.op == QPH_OP_CONV && conv_is_pointwise(q.ws, q.cp) && xs[2] == 1 &&
+        xs[3] == 1 && q.in2 < 0 && q.res_up == 0 && (q.y_ctotal == 0 || q.y_ctotal == q.ws[0]) &&
+        q.y_coff == 0 && q.y_up <= 1 && !net->cl_out[i] && q.ws[0] % 4 == 0 &&
+        linear_nt_eligible(xs[0], q.ws[0], q.ws[1], q.ws[1]))
+      net->cl_pw[i] = true;
+    i += step + (size_t)net->absorb_after[i + step - 1];
+  }
+}
+
 static int run_fpn(qph_net* net, size_t i) {
   hipStream_t s = net->ctx->stream;
   const qph_node* q[4] = {&net->nodes[i], &net->nodes[i + 1], &net->nodes[i + 2],
@@ -1290,6 +1320,7 @@ QPH_API int qph_net_create(qph_ctx* ctx, const qph_net_spec* spec,
     if (rc) return bail(rc);
     rc = plan_fpn(net);
     if (rc) return bail(rc);
+    plan_single_pixel(net);
   }
   rc = hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
   if (rc) return bail(rc);
@@ -1347,14 +1378,8 @@ QPH_API int qph_net_plan(qph_net* net, int32_t* first, int32_t* nodes, int32_t* 
   int32_t n = 0;
   const size_t nn = net->nodes.size();
   for (size_t i = 0; i < nn; n++) {
-    size_t step = 1;
-    int32_t nk = 1;
-    if (net->group_len[i] > 1) step = (size_t)net->group_len[i];
-    else if (net->head[i]) step = 2, nk = net->head_split[i].wp ? 3 : 2;
-    else if (net->fused[i]) step = net->dwpw[i].stem ? 3 : 2;
-    else if (net->convt_fused[i]) step = 2;
-    else if (net->qa_fused[i]) step = 2;
-    else if (net->fpn[i]) step = 4, nk = 3;
+    size_t step = launch_nodes(net, i);
+    const int32_t nk = net->head[i] ? (net->head_split[i].wp ? 3 : 2) : net->fpn[i] ? 3 : 1;
     step += (size_t)net->absorb_after[i + step - 1];
     if (n < cap) {
       if (first) first[n] = (int32_t)i;

@@ -36,3 +36,50 @@ def test_session_linear_tiles(gpu, oracle, rows, k, n, form):
     got = sess.run(x)[0]
     sess.close()
     assert_bitexact(got, onets.run_graph(g, x)[0], f"linear {rows}x{k}x{n} {form}")
+
+
+@pytest.mark.parametrize("n,c,m", [(1, 64, 8), (1, 256, 1280), (2, 256, 1280), (33, 1280, 64),
+                                   (3, 64, 6), (2, 96, 32), (1, 1024, 204)])
+def test_session_single_pixel_conv(gpu, oracle, n, c, m):
+    """1x1 convs of single-pixel maps over the batch, with the bias rules of one
+    item (seeded from 2e5 products on) and of several, and the shapes that stay
+    a GEMM per item (M % 4, C % 64)."""
+    from qppocr_amd import _lib, nets
+    from oracle import nets as onets
+    rng = np.random.default_rng(n * c + m)
+    g = nets.Graph((n, c, 1, 1))
+    w = g.weight((rng.standard_normal((m, c, 1, 1)) / np.sqrt(c)).astype(np.float32))
+    b = g.weight(rng.standard_normal(m).astype(np.float32))
+    g.outputs = [g.conv(0, w, b, act=_lib.ACT_HARDSWISH)]
+    x = rng.standard_normal((n, c, 1, 1)).astype(np.float32)
+    print(f"1x1 conv {n} x {c} -> {m}", flush=True)
+    sess = nets.HipSession(g)
+    for k in {n, 1}:      # every item, and one with the rest padding
+        got = sess.run(x[:k])[0]
+        g1 = nets.Graph((k, c, 1, 1))
+        g1.weights = g.weights
+        g1.outputs = [g1.conv(0, w, b, act=_lib.ACT_HARDSWISH)]
+        assert_bitexact(got, onets.run_graph(g1, x[:k])[0], f"1x1 conv {k} of {n}")
+    sess.close()
+
+
+@pytest.mark.parametrize("rows", [1280, 1159, 1153, 577])
+def test_session_wide_linear_rows(gpu, oracle, rows):
+    """The one-wave GEMM's row stores with a partial last row block."""
+    from qppocr_amd import nets
+    from oracle import nets as onets
+    rng = np.random.default_rng(rows)
+    k, n = 32, 18709 if rows == 577 else 9001
+    g = nets.Graph((rows, 1, 1, k))
+    w = g.weight((rng.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32))
+    logits = g.linear(0, w, g.weight(rng.standard_normal(n).astype(np.float32)))
+    g.outputs = list(g.softmax_argmax(logits, n))
+    x = rng.standard_normal((rows, 1, 1, k)).astype(np.float32)
+    print(f"wide linear {rows} x {k} x {n}", flush=True)
+    sess = nets.HipSession(g)
+    got = sess.run(x)
+    sess.close()
+    ref = onets.run_graph(g, x)
+    assert_bitexact(got[0], ref[0], f"probabilities {rows}x{n}")
+    assert (np.ascontiguousarray(got[1]).view(np.uint32) ==
+            np.ascontiguousarray(ref[1]).view(np.uint32)).all()
