@@ -64,6 +64,9 @@ struct DwPwK {
   int ct;            // halo row pitch: 15 * sw + kw rounded up to 4
   int ctr;           // halo columns read from the image: 15 * sw + kw
   int tiles_x;       // 16-pixel tiles per output row
+  int gpr;           // dwpw_reg_kernel: four-pixel groups per output row,
+  unsigned gmagic;   // and 2^32 / gpr rounded up (a group's row by __umulhi), 0: one
+                     // group a row
   int slices;        // 64-channel slices of M
   int halo, wrows;   // LDS floats of the halo and of the weight slice
   int wdl_pad;       // LDS floats of the depthwise weights (rounded to 64)
@@ -613,61 +616,88 @@ __global__ __launch_bounds__(256) void dwpw_kernel(DwPwK p) {
   }
 }
 
-// Register-fed form of the same block, for the 16-byte path's shapes with
-// C = 4 NS channels (NS = 4, 8, 16 or 32): the same tile (16 output pixels of a
-// row, a 64-channel slice of M) and the same arithmetic, with only the
-// depthwise outputs in LDS (C x 16 floats, at most 8 KB, where dwpw_kernel
-// stages the whole input halo and weight slice: 40-115 KB).  A workgroup
-// this small fits beside other kernels' workgroups on a CU, for instance
-// beside the rec head GEMM (144 KB of LDS a CU) when the det and rec graphs
-// run concurrently.
-//  - First, each lane loads its NS pointwise A operands W[k = 4 s + g][m]
-//    (the k-major repack, m = this wave's 16-channel block + l16) into
-//    registers; their latency runs under the depthwise phase.
-//  - Depthwise: task (channel ci, quarter part) computes the 4 outputs
-//    part * 4 .. + 3 of the tile for channel ci.  Its window is the KH input
-//    rows x 3 aligned 16-byte chunks starting 4 columns left of its first
-//    output's first tap (so the first tap sits SHIFT = 4 - KW / 2 words in),
-//    loaded straight into registers; a chunk is wholly inside or outside
-//    the image (width % 4 == 0), outside ones read 0 through the buffer
-//    range check, which is the zero padding.  The taps and bias come from
-//    memory.  Lanes 4 ci + part: one load instruction touches 16 channels'
-//    rows, four consecutive chunks each.  acc = fma(w, x, acc) over ky then
-//    kx from 0, + bias, activation; outputs past the image store 0.
+// Register-fed form of the same block, for C = 4 NS channels (NS = 4, 8, 16 or 32)
+// and left padding KW / 2: the same arithmetic with only the depthwise outputs
+// in LDS (C x 16 PB floats, where dwpw_kernel stages the whole input halo and
+// weight slice: 40-115 KB).  A workgroup this small fits beside other kernels'
+// workgroups on a CU, for instance beside the rec head when the det and rec
+// graphs run concurrently.
+//  - A tile is PB blocks of 16 output pixels: 4 PB groups of four adjacent
+//    pixels of a row, the groups of an image numbered row by row (so a row of
+//    20 or 26 pixels leaves no more than three slots empty).  blockDim / 64 =
+//    PB x (16-channel blocks of the workgroup's slice of M) waves.
+//  - First, each lane loads its NS pointwise A operands W[m][k = 4 s + g] (m =
+//    this wave's 16-channel block + l16) into registers; their latency runs
+//    under the depthwise phase.  The weight is repacked for it
+//    (dwpw_lane_kernel): four steps of a lane are one 16-byte load.
+//  - Depthwise: task (channel ci, group) computes the group's 4 outputs for
+//    channel ci, from KH input rows loaded straight into registers.  WIDE
+//    (width % 4 == 0, 16-byte aligned): three aligned 16-byte chunks a row
+//    starting 4 columns left of the first output's window centre, each
+//    wholly inside or outside the image.  Otherwise one word a column.  What is
+//    outside reads 0 through the buffer range check, which is the zero
+//    padding.  acc = fma(w, x, acc) over ky then kx from 0, + bias,
+//    activation; slots past the row or the image store 0.
 //  - One barrier; each wave then runs the chain of its 16 output channels
 //    over k = 4 s + g ascending on v_mfma_f32_16x16x4f32, the B operands
 //    read from LDS, and stores as dwpw_kernel does.
 #define DWPW_REG_MAXC 128
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int KH, int KW, int SW, int NS, int AK>
-__global__ __launch_bounds__(256) void dwpw_reg_kernel(DwPwK p) {
+// w[m][c] -> per 16-channel block and group of four steps, the 64 lanes' four A
+// operands (lane (g, l16): channel l16 of the block, k = 4 s + g); 0 past m.
+__global__ __launch_bounds__(256) void dwpw_lane_kernel(const float* __restrict__ w, int m, int c,
+                                                        float* __restrict__ wl) {
+  const int idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (m + 15) / 16 * 16 * c) return;
+  const int j = idx & 3, lane = (idx >> 2) & 63, q = idx >> 8;   // q = block * c / 16 + group
+  const int mb = q / (c / 16), k = 4 * (4 * (q - mb * (c / 16)) + j) + (lane >> 4);
+  const int mo = mb * 16 + (lane & 15);
+  wl[idx] = mo < m ? w[(int64_t)mo * c + k] : 0.0f;
+}
+
+int launch_dwpw_lane_weights(const float* w, int64_t m, int64_t c, float* wl, hipStream_t s) {
+  hipLaunchKernelGGL(dwpw_lane_kernel, dim3(ceil_div(ceil_div(m, 16) * 16 * c, 256)), dim3(256), 0,
+                     s, w, (int)m, (int)c, wl);
+  return launch_check("dwpw_lane_kernel");
+}
+#define DWPW_REG_WAVES 8
+#define DWPW_REG_WGS 512     // workgroups that larger tiles must leave
+
+template <int KH, int KW, int SW, int NS, int AK, int PB, bool WIDE>
+__global__ __launch_bounds__(64 * DWPW_REG_WAVES) void dwpw_reg_kernel(DwPwK p) {
   constexpr int C = 4 * NS;
-  constexpr int PX = 4;
-  constexpr int SHIFT = 4 - KW / 2;
-  constexpr int NC = SHIFT + (PX - 1) * SW + KW;
+  constexpr int PX = 4, G = 4 * PB, P = 16 * PB;   // pixels a task, groups and pixels a tile
+  constexpr int SHIFT = WIDE ? 4 - KW / 2 : 0;     // window column of the first tap
+  constexpr int NC = SHIFT + (PX - 1) * SW + KW;   // window columns
   constexpr int NV = (NC + 3) / 4;
-  static_assert(C <= DWPW_REG_MAXC && NV == 3, "");
-  __shared__ __attribute__((aligned(16))) float t[C * 16];
-  const int tid = threadIdx.x, lane = tid & 63;
+  static_assert(C <= DWPW_REG_MAXC && (!WIDE || NV == 3), "");
+  __shared__ __attribute__((aligned(16))) float t[C * P];
+  const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
-  const int img = blockIdx.z, slice = blockIdx.y;
-  const int oy = blockIdx.x / p.tiles_x;
-  const int ox0 = (blockIdx.x - oy * p.tiles_x) * 16;
-  const int mb = slice * 4 + wave;            // 16-channel block index
+  const int img = blockIdx.z;
+  const int pb = wave % PB;                                   // this wave's pixel block
+  const int mb = blockIdx.y * (nt / (64 * PB)) + wave / PB;   // and 16-channel block
   const unsigned OOB = 0x80000000u;
+  // group -> output row and first column (groups * per row < 2^32)
+  const int g0 = blockIdx.x * G;
+  auto place = [&](int g, int& oy, int& ox) {
+    oy = p.gmagic ? (int)__umulhi((unsigned)g, p.gmagic) : g;
+    ox = 4 * (g - oy * p.gpr);
+  };
 
-  // pointwise A operands and this lane's four bias terms, issued first
+  // pointwise A operands (four steps a load) and this lane's four bias terms,
+  // issued first
   float wa[NS];
-  {
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)p.wk, 0, C * p.mpad * 4, 0x00020000);
-    const int col = mb * 16 + l16;
-    const unsigned vo = col < p.mpad ? (unsigned)(lg * p.mpad + col) * 4u : OOB;
+  if (mb * 16 < p.m) {
+    const f32x4* wl = (const f32x4*)p.wk + (int64_t)mb * (NS / 4) * 64 + lane;
 #pragma unroll
-    for (int s = 0; s < NS; s++)
-      wa[s] = __builtin_bit_cast(
-          float, __builtin_amdgcn_raw_buffer_load_b32(wr, vo, 16 * s * p.mpad, 0));
+    for (int s = 0; s < NS / 4; s++) {
+      const f32x4 q = wl[s * 64];
+#pragma unroll
+      for (int j = 0; j < 4; j++) wa[4 * s + j] = q[j];
+    }
   }
   float bpre[4];
 #pragma unroll
@@ -681,34 +711,52 @@ __global__ __launch_bounds__(256) void dwpw_reg_kernel(DwPwK p) {
     const int64_t plane = (int64_t)p.h * p.w;
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(p.x + (int64_t)img * C * plane), 0, (int)(C * plane * 4), 0x00020000);
-    const int iy0 = oy * p.sh - p.ph;
-#pragma unroll
-    for (int e0 = 0; e0 < 4 * C; e0 += 256) {
-      const int e = e0 + tid;
-      if (4 * C % 256 != 0 && e >= 4 * C) break;
-      const int ci = e >> 2, part = e & 3;
-      const int px0 = part * PX;
-      const int wx = (ox0 + px0) * SW - 4;    // window column 0 (a multiple of 4)
+    for (int e = tid; e < C * G; e += nt) {
+      const int ci = e / G, part = e % G;
+      int oy, ox;
+      place(g0 + part, oy, ox);
+      const bool gok = oy < p.oh;   // (groups past the image: nothing read, 0 stored)
+      const int iy0 = oy * p.sh - p.ph;
+      const int wx = ox * SW - (WIDE ? 4 : KW / 2);    // window column 0
       float r[KH][4 * NV];
 #pragma unroll
       for (int ky = 0; ky < KH; ky++) {
         const int iy = iy0 + ky;
-        const bool rok = iy >= 0 && iy < p.h;
+        const bool rok = gok && iy >= 0 && iy < p.h;
+        const int base = ci * (int)plane + iy * p.w;
+        if constexpr (WIDE) {
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
-          const int ix = wx + 4 * v;
-          const unsigned off =
-              rok && ix >= 0 && ix < p.w ? (unsigned)((ci * (int)plane + iy * p.w + ix) * 4) : OOB;
-          const f32x4 q =
-              __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, 0));
+          for (int v = 0; v < NV; v++) {
+            const int ix = wx + 4 * v;
+            const unsigned off =
+                rok && ix >= 0 && ix < p.w ? (unsigned)((base + ix) * 4) : OOB;
+            const f32x4 q =
+                __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, 0));
 #pragma unroll
-          for (int j = 0; j < 4; j++) r[ky][4 * v + j] = q[j];
+            for (int j = 0; j < 4; j++) r[ky][4 * v + j] = q[j];
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < NC; j++) {
+            const int ix = wx + j;
+            const unsigned off =
+                rok && ix >= 0 && ix < p.w ? (unsigned)((base + ix) * 4) : OOB;
+            r[ky][j] =
+                __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, off, 0, 0));
+          }
         }
       }
+      // the channel's taps, four a load (4-byte aligned)
       float wv[KH * KW];
       const float* wp = p.wd + ci * KH * KW;
 #pragma unroll
-      for (int j = 0; j < KH * KW; j++) wv[j] = wp[j];
+      for (int j = 0; j + 4 <= KH * KW; j += 4) {
+        const f32x4_a4 q = *(const f32x4_a4*)(wp + j);
+#pragma unroll
+        for (int u = 0; u < 4; u++) wv[j + u] = q[u];
+      }
+      wv[KH * KW - 1] = wp[KH * KW - 1];
+      static_assert(KH * KW % 4 == 1, "");
       const float bdv = p.bd ? p.bd[ci] : 0.0f;
       float acc[PX];
 #pragma unroll
@@ -724,21 +772,24 @@ __global__ __launch_bounds__(256) void dwpw_reg_kernel(DwPwK p) {
 #pragma unroll
       for (int q = 0; q < PX; q++) {
         const float v = act_k<AK>(acc[q] + bdv, p.act_d);
-        o[q] = ox0 + px0 + q < p.ow ? v : 0.0f;
+        o[q] = gok && ox + q < p.ow ? v : 0.0f;
       }
-      *(f32x4*)(t + ci * 16 + px0) = f32x4{o[0], o[1], o[2], o[3]};
+      *(f32x4*)(t + ci * P + part * PX) = f32x4{o[0], o[1], o[2], o[3]};
     }
   }
   __syncthreads();
 
-  // pointwise chain of this wave's 16 channels
+  // pointwise chain of this wave's 16 channels and 16 pixels
   if (mb * 16 >= p.m) return;
   const int npx = p.oh * p.ow;
-  const int px = oy * p.ow + ox0 + l16;
-  const bool pok = ox0 + l16 < p.ow;
+  int py, pxc;
+  place(g0 + 4 * pb + (l16 >> 2), py, pxc);
+  pxc += l16 & 3;
+  const int px = py * p.ow + pxc;
+  const bool pok = py < p.oh && pxc < p.ow;
   float bv[NS];
 #pragma unroll
-  for (int s = 0; s < NS; s++) bv[s] = t[(4 * s + lg) * 16 + l16];
+  for (int s = 0; s < NS; s++) bv[s] = t[(4 * s + lg) * P + 16 * pb + l16];
   f32x4 acc;
 #pragma unroll
   for (int v = 0; v < 4; v++) {
@@ -862,26 +913,62 @@ static bool dwpw_vec(const DwPwArgs& a) {
          (!a.bd || al(a.bd)) && al(a.wk);
 }
 
-// the register-fed form: the 16-byte path with C = 16, 32, 64 or 128
-static bool dwpw_reg_ok(const DwPwArgs& a) {
-  return a.c == 16 || a.c == 32 || a.c == 64 || a.c == 128;
+// the register-fed form: C = 16, 32, 64 or 128, left padding KW / 2
+bool dwpw_lane_weights(const DwPwArgs& a) {
+  const int64_t gpr = (a.ow + 3) / 4;
+  return (a.c == 16 || a.c == 32 || a.c == 64 || a.c == 128) && !a.stem && a.pw == a.kw / 2 &&
+         (a.oh * gpr + 64) * gpr < (1ll << 32);
+}
+
+template <int KH, int KW, int SW, int NS, int AK, int PB>
+static void launch_dwpw_reg_w(bool wide, dim3 grid, dim3 block, const DwPwK& p, hipStream_t s) {
+  if (wide)
+    hipLaunchKernelGGL((dwpw_reg_kernel<KH, KW, SW, NS, AK, PB, true>), grid, block, 0, s, p);
+  else
+    hipLaunchKernelGGL((dwpw_reg_kernel<KH, KW, SW, NS, AK, PB, false>), grid, block, 0, s, p);
+}
+
+template <int KH, int KW, int SW, int NS, int AK>
+static void launch_dwpw_reg_p(int pb, bool wide, dim3 grid, dim3 block, const DwPwK& p,
+                              hipStream_t s) {
+  if (pb == 4) launch_dwpw_reg_w<KH, KW, SW, NS, AK, 4>(wide, grid, block, p, s);
+  else if (pb == 2) launch_dwpw_reg_w<KH, KW, SW, NS, AK, 2>(wide, grid, block, p, s);
+  else launch_dwpw_reg_w<KH, KW, SW, NS, AK, 1>(wide, grid, block, p, s);
 }
 
 template <int KH, int KW, int SW, int NS>
-static int launch_dwpw_reg_t(dim3 grid, const DwPwK& p, hipStream_t s) {
+static int launch_dwpw_reg_t(int64_t n, DwPwK& p, bool wide, hipStream_t s) {
+  // The slice's channel blocks and the tile's pixel blocks share up to eight
+  // waves.  Eight channel blocks a workgroup halve the depthwise work of 128
+  // channels (each slice of M repeats it): at 1536 x 1536 the 96 x 96 blocks take
+  // 14.4-16.4 us instead of 17.2-19.9.  Below 256 workgroups the launches are
+  // bound by latency and slices of four spread over more CUs (a 160 x 416 det
+  // pass 135.3 us, 137.2 with eight).  Tiles of 32 and 64 pixels fill the waves
+  // where M is small (384 x 384 x 32 25.7 -> 21.5 us), if 512 workgroups are left.
+  const int mbs = (p.m + 15) / 16;
+  const int64_t groups = (int64_t)p.oh * p.gpr;
+  auto wgs = [&](int mw, int pb) { return (int64_t)ceil_div(groups, 4 * pb) * ceil_div(mbs, mw) * n; };
+  int mw = std::min(mbs, DWPW_REG_WAVES), pb = 1;
+  if (wgs(mw, 1) < 256) mw = std::min(mbs, 4);
+  while (2 * pb * mw <= DWPW_REG_WAVES && pb < 4 && wgs(mw, 2 * pb) >= DWPW_REG_WGS) pb *= 2;
+  const dim3 grid((unsigned)ceil_div(groups, 4 * pb), (unsigned)ceil_div(mbs, mw), (unsigned)n);
+  const dim3 block((unsigned)(64 * mw * pb));
   if (p.act_d.kind == 3 && p.act_p.kind == 3)
-    hipLaunchKernelGGL((dwpw_reg_kernel<KH, KW, SW, NS, 3>), grid, dim3(256), 0, s, p);
+    launch_dwpw_reg_p<KH, KW, SW, NS, 3>(pb, wide, grid, block, p, s);
   else
-    hipLaunchKernelGGL((dwpw_reg_kernel<KH, KW, SW, NS, 0>), grid, dim3(256), 0, s, p);
+    launch_dwpw_reg_p<KH, KW, SW, NS, 0>(pb, wide, grid, block, p, s);
   return launch_check("dwpw_reg_kernel");
 }
 
 template <int KH, int KW, int SW>
-static int launch_dwpw_reg(int64_t c, dim3 grid, const DwPwK& p, hipStream_t s) {
-  if (c == 16) return launch_dwpw_reg_t<KH, KW, SW, 4>(grid, p, s);
-  if (c == 32) return launch_dwpw_reg_t<KH, KW, SW, 8>(grid, p, s);
-  if (c == 64) return launch_dwpw_reg_t<KH, KW, SW, 16>(grid, p, s);
-  return launch_dwpw_reg_t<KH, KW, SW, 32>(grid, p, s);
+static int launch_dwpw_reg(const DwPwArgs& a, DwPwK& p, hipStream_t s) {
+  p.gpr = (int)((a.ow + 3) / 4);
+  p.gmagic = p.gpr == 1 ? 0u : (unsigned)(((1ull << 32) + p.gpr - 1) / p.gpr);
+  const bool wide = a.w % 4 == 0 && ((uintptr_t)a.x & 15) == 0;
+  if (a.c == 16) return launch_dwpw_reg_t<KH, KW, SW, 4>(a.n, p, wide, s);
+  if (a.c == 32) return launch_dwpw_reg_t<KH, KW, SW, 8>(a.n, p, wide, s);
+  if (a.c == 64) return launch_dwpw_reg_t<KH, KW, SW, 16>(a.n, p, wide, s);
+  return launch_dwpw_reg_t<KH, KW, SW, 32>(a.n, p, wide, s);
 }
 
 bool dwpw_stem_eligible(const DwPwArgs& a) {
@@ -959,10 +1046,10 @@ int launch_dwpw(const DwPwArgs& a, hipStream_t s) {
     if (px == 2) return launch_dwpw_t<3, 3, 2, 2, true, false, 1>(grid, lds, p, s);
     return launch_dwpw_t<3, 3, 2, 1, true, false, 1>(grid, lds, p, s);
   }
-  if (dwpw_vec(a) && dwpw_reg_ok(a)) {
-    if (a.kh == 5) return launch_dwpw_reg<5, 5, 1>(a.c, grid, p, s);
-    if (a.sw == 1) return launch_dwpw_reg<3, 3, 1>(a.c, grid, p, s);
-    return launch_dwpw_reg<3, 3, 2>(a.c, grid, p, s);
+  if (dwpw_lane_weights(a)) {
+    if (a.kh == 5) return launch_dwpw_reg<5, 5, 1>(a, p, s);
+    if (a.sw == 1) return launch_dwpw_reg<3, 3, 1>(a, p, s);
+    return launch_dwpw_reg<3, 3, 2>(a, p, s);
   }
   // the 16-byte path's halo: whole chunks, channels contiguous
   const int vch = a.kh == 5 ? VecGeom<5, 5, 1>::CH : a.sw == 1 ? VecGeom<3, 3, 1>::CH

@@ -310,7 +310,7 @@ struct DwPwArgs {
   const float* wd; const float* bd;
   int64_t kh, kw, sh, sw, ph, pw, oh, ow;
   Act act_d;
-  const float* wk; const float* bp;
+  const float* wk; const float* bp;   // (wk: see dwpw_lane_weights)
   int64_t m;
   int seed_rule;
   Act act_p;
@@ -336,6 +336,10 @@ bool dwpw_eligible(const DwPwArgs& a);
 // the stem conv that can run inside the dw + pw launch of a (3 -> a.c
 // channels, 3x3, stride 2, pad 1, into a 3x3 stride-2 pad-1 depthwise)
 bool dwpw_stem_eligible(const DwPwArgs& a);
+// true: a.wk is the 1x1 weight as launch_dwpw_lane_weights lays it out
+// (ceil(m / 16) 16 c floats), not the k-major repack
+bool dwpw_lane_weights(const DwPwArgs& a);
+int launch_dwpw_lane_weights(const float* w, int64_t m, int64_t c, float* wl, hipStream_t s);
 int launch_dwpw(const DwPwArgs& a, hipStream_t s);
 // 3x3 convs the direct kernel takes; up to four independent ones in one launch
 bool direct3x3_eligible(const ConvArgs& a);

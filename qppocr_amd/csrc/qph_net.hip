@@ -654,7 +654,10 @@ static int plan_dwpw(qph_net* net) {
     QPH_TRY(hip_check(hipMalloc((void**)&wk, (size_t)dense_conv_wk_floats(f.m, f.c, 1, 1) * 4),
                       "hipMalloc(repacked 1x1 weight)"));
     net->wk[i + 1] = wk;
-    QPH_TRY(launch_repack_conv_w_taps(net->weights[q.w], f.m, f.c, 1, wk, net->ctx->stream));
+    if (dwpw_lane_weights(f))
+      QPH_TRY(launch_dwpw_lane_weights(net->weights[q.w], f.m, f.c, wk, net->ctx->stream));
+    else
+      QPH_TRY(launch_repack_conv_w_taps(net->weights[q.w], f.m, f.c, 1, wk, net->ctx->stream));
     f.wk = wk;
     net->dwpw[at] = f;
     net->fused[at] = true;
