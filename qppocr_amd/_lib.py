@@ -26,6 +26,7 @@ NET_FUSED_HEAD = 2
 NOALLOC_WK_FLOATS = 1 << 20
 
 I64 = ctypes.c_int64
+I64_4 = I64 * 4
 I32 = ctypes.c_int32
 F32 = ctypes.c_float
 P = ctypes.c_void_p
