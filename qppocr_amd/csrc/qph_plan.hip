@@ -69,6 +69,14 @@ enum {
 __device__ __forceinline__ unsigned real_n(const float* arena) {
   return *(const unsigned*)arena;
 }
+// Whether image b lies past the real batch (arena word 0; 0: every image is
+// real).  The first image never does, so its workgroups start without that
+// load, a cold round trip in front of everything else a kernel reads.
+__device__ __forceinline__ bool past_image(const float* arena, int64_t b) {
+  if (b == 0) return false;
+  const unsigned rn = real_n(arena);
+  return rn != 0 && b >= (int64_t)rn;
+}
 
 __device__ __forceinline__ float4 act4(float4 v, const Act& a) {
   return make_float4(act_apply(v.x, a), act_apply(v.y, a), act_apply(v.z, a), act_apply(v.w, a));
@@ -86,8 +94,7 @@ __global__ __launch_bounds__(256) void plan_entry_kernel(EntryK p) {
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= p.nb * p.hw) return;
   const int64_t n = gid / p.hw, pos = gid - n * p.hw;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && n >= rn) return;
+  if (past_image(p.arena, n)) return;
   const float* xn = p.x + n * p.c * p.hw + pos;
   float4* yo = (float4*)p.y + gid * p.cp4;
   for (int64_t c4 = 0; c4 < p.cp4; c4++) {
@@ -268,8 +275,7 @@ constexpr int CONV_CS = 8;  // k-steps (4 k each) loaded per batch
 // keeps every region below 2^31 words).
 __global__ __launch_bounds__(256) void plan_conv_kernel(ConvK p) {
   const int b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && (unsigned)b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int N = (int)p.N, P = (int)p.P, ow = (int)p.ow;
@@ -380,8 +386,7 @@ constexpr int CONV_LDS_SLOTS = (CONV_LDS_TAPS * 32 + 63) / 64;  // quads per lan
 __global__ __launch_bounds__(256) void plan_conv_lds_kernel(ConvK p) {
   extern __shared__ float4 patches[];  // per wave [taps][32]
   const int b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && (unsigned)b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int wave = (int)blockIdx.x * 4 + wv;
   const int N = (int)p.N, P = (int)p.P, ow = (int)p.ow;
@@ -552,8 +557,7 @@ __global__ __launch_bounds__(64) void plan_conv_dma_kernel(ConvK p) {
   using G = DmaGeom<TAPS>;
   extern __shared__ float4 ring[];  // CONV_DMA_D buffers of G::BUF float4
   const int b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && (unsigned)b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int lane = threadIdx.x;
   const int N = (int)p.N, P = (int)p.P, ow = (int)p.ow;
   const int ncob = (N + 15) >> 4;
@@ -673,8 +677,7 @@ template <int SW, int NCB>
 __global__ __launch_bounds__(256) void plan_stem_kernel(ConvK p) {
   __shared__ float4 patches[4][9 * 32];
   const int b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && (unsigned)b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int wave = (int)blockIdx.x * 4 + wv;
   const int N = (int)p.N, P = (int)p.P, ow = (int)p.ow;
@@ -832,8 +835,7 @@ __device__ __forceinline__ void plan_conv_halo_tile(const ConvK& p, int tiles_x,
   using G = HaloGeom<SW, NCB>;
   constexpr int L = G::L;
   const int b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && (unsigned)b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = wave / NCB, ub = wave - row * NCB, co0 = ub * 16;
@@ -1091,8 +1093,7 @@ struct DwK {
 };
 __global__ __launch_bounds__(256) void plan_dw_kernel(DwK p) {
   const int64_t b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= p.P * p.c4) return;
   const int64_t c4 = gid % p.c4, m = gid / p.c4;
@@ -1118,48 +1119,74 @@ __global__ __launch_bounds__(256) void plan_dw_kernel(DwK p) {
   ((float4*)p.y)[b * p.P * p.c4 + gid] = o;
 }
 
-// The same depthwise with 4 adjacent output pixels of one channel quad per
-// thread (KH x KW taps, x-stride SW, any y-stride): the taps' weight quads
-// sit in registers and each input row's 3 SW + KW quads are read once for
-// the 4 outputs; threads run channel quads fastest (16-byte loads and stores
-// of consecutive lanes are contiguous).  Each output's chain is plan_dw_kernel's.
-template <int KH, int KW, int SW>
+// The same depthwise with PX adjacent output pixels of one channel quad per
+// thread (KH x KW taps, x-stride SW, any y-stride): each input row's
+// (PX - 1) SW + KW quads are read once for the PX outputs; threads run channel
+// quads fastest (16-byte loads and stores of consecutive lanes are
+// contiguous).  Each output's chain is plan_dw_kernel's.  Most launches are
+// bound by latency: the inputs and weights of the whole window go out
+// together, as bounds-checked buffer loads (a tap outside the image reads 0)
+// at 32-bit offsets, from as many threads as the map allows.  3x3 runs one
+// pixel a thread (four measured 7.5 against 4.8 us on a 320x320 map of 16
+// channels, and 19.0 against 15.5 on 768x768), 5x5 two (one: the same on
+// 40x40x128, 11.9 against 10.0 us on 96x96).  The eleven depthwise launches
+// of a 640x640 page: 86 us with four pixels a thread, 64-bit index arithmetic
+// and a load a row, 51 as they are.
+template <int KH, int KW, int SW, int PX>
 __global__ __launch_bounds__(256) void plan_dw_px_kernel(DwK p) {
-  constexpr int NC = 3 * SW + KW;   // input columns a thread reads per row
-  const int64_t b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && b >= rn) return;
-  const int64_t ngx = (p.ow + 3) / 4;
-  const int64_t oh = p.P / p.ow;
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= oh * ngx * p.c4) return;
-  const int64_t c4 = gid % p.c4, m = gid / p.c4;
-  const int64_t oy = m / ngx, ox0 = (m - oy * ngx) * 4;
-  const float4* xb = (const float4*)p.x + b * p.ih * p.iw * p.c4;
-  const float4* w4 = (const float4*)p.w;
+  constexpr int NC = (PX - 1) * SW + KW;   // input columns a thread reads per row
+  const int b = blockIdx.y;
+  if (past_image(p.arena, b)) return;
+  const unsigned c4n = (unsigned)p.c4, ow = (unsigned)p.ow, ngx = (ow + PX - 1) / PX;
+  const unsigned oh = (unsigned)p.P / ow;
+  const unsigned gid = blockIdx.x * blockDim.x + threadIdx.x;
+  if (gid >= oh * ngx * c4n) return;
+  const unsigned m = gid / c4n, c4 = gid - m * c4n;
+  const unsigned oy = m / ngx, ox0 = (m - oy * ngx) * PX;
+  const int ih = (int)p.ih, iw = (int)p.iw;
+  // offsets past the map: each alone is beyond the largest map (2^30 bytes),
+  // and their sum does not wrap
+  const unsigned NOROW = 0x40000000u, NOCOL = 0x80000000u;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.x + (size_t)b * ih * iw * c4n * 4), 0, ih * iw * (int)c4n * 16, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.w, 0, KH * KW * (int)c4n * 16, 0x00020000);
   float4 wv[KH * KW];
 #pragma unroll
-  for (int t = 0; t < KH * KW; t++) wv[t] = w4[t * p.c4 + c4];
-  float4 acc[4];
+  for (int t = 0; t < KH * KW; t++)
+    wv[t] = __builtin_bit_cast(
+        float4, __builtin_amdgcn_raw_buffer_load_b128(wr, c4 * 16u, t * c4n * 16u, 0));
+  unsigned col[NC];
 #pragma unroll
-  for (int q = 0; q < 4; q++) acc[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int cc = 0; cc < NC; cc++) {
+    const int ix = (int)ox0 * SW - (int)p.pl + cc;
+    col[cc] = (unsigned)ix < (unsigned)iw ? ((unsigned)ix * c4n + c4) * 16u : NOCOL;
+  }
+  float4 xv[KH][NC];
 #pragma unroll
   for (int ky = 0; ky < KH; ky++) {
-    const int64_t iy = oy * p.sh - p.pt + ky;
-    const bool rok = iy >= 0 && iy < p.ih;
-    float4 xv[NC];
+    const int iy = (int)oy * (int)p.sh - (int)p.pt + ky;
+    const unsigned row =
+        (unsigned)iy < (unsigned)ih ? (unsigned)iy * (unsigned)iw * c4n * 16u : NOROW;
 #pragma unroll
-    for (int cc = 0; cc < NC; cc++) {
-      const int64_t ix = ox0 * SW - p.pl + cc;
-      xv[cc] = (rok && ix >= 0 && ix < p.iw) ? xb[(iy * p.iw + ix) * p.c4 + c4]
-                                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
+    for (int cc = 0; cc < NC; cc++)
+      xv[ky][cc] = __builtin_bit_cast(
+          float4, __builtin_amdgcn_raw_buffer_load_b128(xr, row + col[cc], 0, 0));
+  }
+  // yc = acc + bv with bv = 0 when there is no bias (conv.rs:461-505)
+  const float4 bv = p.bias ? ((const float4*)p.bias)[c4] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  __builtin_amdgcn_sched_barrier(0);   // every load ahead of the products
+  float4 acc[PX];
+#pragma unroll
+  for (int q = 0; q < PX; q++) acc[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+  for (int ky = 0; ky < KH; ky++) {
 #pragma unroll
     for (int kx = 0; kx < KW; kx++) {
       const float4 w = wv[ky * KW + kx];
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const float4 x = xv[q * SW + kx];
+      for (int q = 0; q < PX; q++) {
+        const float4 x = xv[ky][q * SW + kx];
         acc[q].x = __builtin_fmaf(w.x, x.x, acc[q].x);
         acc[q].y = __builtin_fmaf(w.y, x.y, acc[q].y);
         acc[q].z = __builtin_fmaf(w.z, x.z, acc[q].z);
@@ -1167,16 +1194,24 @@ __global__ __launch_bounds__(256) void plan_dw_px_kernel(DwK p) {
       }
     }
   }
-  // yc = acc + bv with bv = 0 when there is no bias (conv.rs:461-505)
-  const float4 bv = p.bias ? ((const float4*)p.bias)[c4] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    if (ox0 + q >= p.ow) break;
-    const int64_t e = (oy * p.ow + ox0 + q) * p.c4 + c4;
+  for (int q = 0; q < PX; q++) {
+    if (ox0 + q >= ow) break;
+    const size_t e = (size_t)b * (size_t)p.P * c4n + ((oy * ow + ox0 + q) * c4n + c4);
     float4 o = act4(add4(acc[q], bv), p.act);
-    if (p.res) o = add4(o, ((const float4*)p.res)[b * p.P * p.c4 + e]);
-    ((float4*)p.y)[b * p.P * p.c4 + e] = o;
+    if (p.res) o = add4(o, ((const float4*)p.res)[e]);
+    ((float4*)p.y)[e] = o;
   }
+}
+
+template <int K, int SW>
+static void launch_plan_dw_px(const DwK& k, unsigned nb, hipStream_t s) {
+  constexpr int PX = K == 3 ? 1 : 2;
+  const int64_t threads = k.P / k.ow * ((k.ow + PX - 1) / PX) * k.c4;
+  // a launch of few waves is spread over as many CUs as there are waves
+  const unsigned block = threads * nb < (1 << 17) ? 64 : 256;
+  hipLaunchKernelGGL((plan_dw_px_kernel<K, K, SW, PX>),
+                     dim3((unsigned)ceil_div(threads, block), nb), dim3(block), 0, s, k);
 }
 
 // ------------------------------------------------------- conv transpose
@@ -1213,12 +1248,16 @@ __global__ __launch_bounds__(256) void plan_convt_kernel(ConvtK p) {
 // The det head's tail: an n_convt (2x2, stride 2, CI -> CM channels) whose
 // output only a second such n_convt (CM -> at most 4 channels) reads, whose
 // output only an n_exit (NHWC -> NCHW, sigmoid or not) reads, in one pass.
-// A thread takes one pixel of the middle map: its CM channels by
-// plan_convt_kernel's chains (input channels ascending from +0, + bias, the
-// activation), then the 2 x 2 output pixels it feeds (the same chains over
-// the CM channels) through the exit into NCHW.  A block's threads share the
-// tap parity of their middle pixel (blockIdx.y), so every weight a chain
-// reads is the same for the whole block (scalar loads).
+// A wave takes 16 input pixels: the first conv-transpose is a (4 taps x CM)
+// by CI by 16 product on the MFMAs (plan_convt_kernel's chains: input channels
+// ascending from +0), row 4 q + v of M tile mt being channel 4 mt + v of tap
+// q, so that lane (pixel l16, tap g) ends with the CM channels of one middle
+// pixel; after bias and activation the lane runs the 2 x 2 output pixels it
+// feeds (the same chains over the CM channels, the weights in LDS as
+// [channel][output][tap]) through the exit into NCHW.  The work is small and
+// latency bounds it: one round of operand loads a wave.  (A thread per middle
+// pixel with wave-uniform weights through scalar loads waited for some twenty
+// rounds of them: 16.9 us on a 160x160 map, now 11.0.)
 struct ConvtPairK {
   const float* arena;
   const float* x; const float* w1; const float* b1; const float* w2; const float* b2; float* y;
@@ -1229,51 +1268,69 @@ struct ConvtPairK {
 };
 template <int CI, int CM>
 __global__ __launch_bounds__(256) void plan_convt_pair_kernel(ConvtPairK p) {
-  const int b = blockIdx.z, py = blockIdx.y >> 1, px = blockIdx.y & 1;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && (unsigned)b >= rn) return;
-  const int t = (int)blockIdx.x * 256 + (int)threadIdx.x;
-  if (t >= p.h * p.w) return;
-  const int i = t / p.w, j = t - i * p.w;
-  float xv[CI];
-  const float4* xr = (const float4*)(p.x + ((size_t)(b * p.h + i) * p.w + j) * CI);
+  static_assert(CI % 4 == 0 && CM % 4 == 0, "");
+  __shared__ __attribute__((aligned(16))) float sw2[CM * 4 * 4];   // [c][o][tap]
+  const int b = blockIdx.y;
+  if (past_image(p.arena, b)) return;
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
+  const int t0 = (int)blockIdx.x * 64 + (tid >> 6) * 16, hw = p.h * p.w;
+  // operands: a lane past the map repeats the last pixel and stores nothing
+  const int t = min(t0 + l16, hw - 1);
+  const float* xr = p.x + ((size_t)b * hw + t) * CI + lg;
+  const float* w1 = p.w1 + ((l16 >> 2) * CI + lg) * CM + (l16 & 3);   // [tap][ci][CM]
+  float bx[CI / 4], aw[CM / 4][CI / 4];
 #pragma unroll
-  for (int q = 0; q < CI / 4; q++) {
-    const float4 v = xr[q];
-    xv[4 * q] = v.x;
-    xv[4 * q + 1] = v.y;
-    xv[4 * q + 2] = v.z;
-    xv[4 * q + 3] = v.w;
+  for (int s = 0; s < CI / 4; s++) bx[s] = xr[4 * s];
+#pragma unroll
+  for (int mt = 0; mt < CM / 4; mt++)
+#pragma unroll
+    for (int s = 0; s < CI / 4; s++) aw[mt][s] = w1[4 * s * CM + 4 * mt];
+  float b1[CM / 4][4];
+#pragma unroll
+  for (int c = 0; c < CM; c++) b1[c >> 2][c & 3] = p.b1 ? p.b1[c] : 0.0f;
+  for (int e = tid; e < CM * 4 * p.c_out; e += 256) {
+    const int q = e & 3, r = e >> 2, c = r / p.c_out, o = r - c * p.c_out;
+    sw2[(c * 4 + o) * 4 + q] = p.w2[(q * CM + c) * p.co2p + o];   // [tap][c][co2p]
   }
-  const float* w1 = p.w1 + (size_t)(py * 2 + px) * CI * CM;   // [tap][ci][CM]
-  float m[CM];
+  __syncthreads();
+  f32x4 m[CM / 4];
+#pragma unroll
+  for (int mt = 0; mt < CM / 4; mt++) {
+    m[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < CI / 4; s++)
+      m[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[mt][s], bx[s], m[mt], 0, 0, 0);
+  }
 #pragma unroll
   for (int c = 0; c < CM; c++) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int ci = 0; ci < CI; ci++) acc = __builtin_fmaf(xv[ci], w1[ci * CM + c], acc);
-    if (p.b1) acc = acc + p.b1[c];
-    m[c] = act_apply(acc, p.act1);
+    float v = m[c >> 2][c & 3];
+    if (p.b1) v = v + b1[c >> 2][c & 3];
+    m[c >> 2][c & 3] = act_apply(v, p.act1);
   }
+  if (t0 + l16 >= hw) return;
+  const int i = t / p.w, j = t - i * p.w;
   const int H2 = 4 * p.h, W2 = 4 * p.w;
-  const int my = 2 * i + py, mx = 2 * j + px;
+  const int oy = 4 * i + 2 * (lg >> 1), ox = 4 * j + 2 * (lg & 1);
 #pragma unroll
-  for (int qy = 0; qy < 2; qy++)
+  for (int o = 0; o < 4; o++) {
+    if (o >= p.c_out) break;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};   // output (tap >> 1, tap & 1) of the 2 x 2
 #pragma unroll
-    for (int qx = 0; qx < 2; qx++) {
-      const float* w2 = p.w2 + (size_t)(qy * 2 + qx) * CM * p.co2p;   // [tap][c][co2p]
-      const int oy = 2 * my + qy, ox = 2 * mx + qx;
+    for (int c = 0; c < CM; c++) {
+      const f32x4 wv = *(const f32x4*)(sw2 + (c * 4 + o) * 4);
+      const float v = m[c >> 2][c & 3];
 #pragma unroll
-      for (int o = 0; o < 4; o++) {
-        if (o >= p.c_out) break;
-        float acc = 0.0f;
-#pragma unroll
-        for (int c = 0; c < CM; c++) acc = __builtin_fmaf(m[c], w2[c * p.co2p + o], acc);
-        if (p.b2) acc = acc + p.b2[o];
-        acc = act_apply(acc, p.act2);
-        p.y[((size_t)(b * p.c_out + o) * H2 + oy) * W2 + ox] = p.sigmoid ? sigmoid1(acc) : acc;
-      }
+      for (int q = 0; q < 4; q++) acc[q] = __builtin_fmaf(v, wv[q], acc[q]);
     }
+    float* yo = p.y + ((size_t)(b * p.c_out + o) * H2 + oy) * W2 + ox;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      float v = acc[q];
+      if (p.b2) v = v + p.b2[o];
+      v = act_apply(v, p.act2);
+      yo[(size_t)(q >> 1) * W2 + (q & 1)] = p.sigmoid ? sigmoid1(v) : v;
+    }
+  }
 }
 
 // ------------------------------------------------------------------ pool
@@ -1288,8 +1345,7 @@ __device__ __forceinline__ float pool_acc(bool mx, float acc, float t) {
 }
 __global__ __launch_bounds__(256) void plan_pool_kernel(PoolNK p) {
   const int64_t b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= p.P * p.c4) return;
   const int64_t c4 = gid % p.c4, m = gid / p.c4;
@@ -1367,8 +1423,7 @@ __device__ __forceinline__ int resize_src(int o, int in, int out) {
 struct ResizeAddK { const float* arena; const float4* x; const float4* a; float4* y; int P, c4, ow, oh, iw, ih; };
 __global__ __launch_bounds__(256) void plan_resize_add_kernel(ResizeAddK p) {
   const int b = blockIdx.y;
-  const unsigned rn = real_n(p.arena);
-  if (rn != 0 && (unsigned)b >= rn) return;
+  if (past_image(p.arena, b)) return;
   const int gid = (int)blockIdx.x * 256 + (int)threadIdx.x;
   if (gid >= p.P * p.c4) return;
   const int m = gid / p.c4, c4 = gid - m * p.c4;
@@ -2224,14 +2279,16 @@ int decode(Decoder& d, const qph_plan_dispatch& q, std::vector<PendingHw>& pendi
             e.res == OFF_NONE ? nullptr : d.at(e.res), d.at(e.y),
             P, C / 4, ow, iw, ih, taps, kw, sh, sw, pt, pl_, e.act};
       const int64_t kh = taps / kw;
-      if (((kh == 3 && kw == 3) || (kh == 5 && kw == 5)) && (sw == 1 || sw == 2)) {
-        const int64_t threads = (P / ow) * ((ow + 3) / 4) * (C / 4);
-        return add_launch(pl, d.idx, [k, nb, threads, kh, sw](hipStream_t s) {
-          const dim3 grid(blocks_for(threads), (unsigned)nb);
-          if (kh == 3 && sw == 1) hipLaunchKernelGGL((plan_dw_px_kernel<3, 3, 1>), grid, dim3(256), 0, s, k);
-          else if (kh == 3) hipLaunchKernelGGL((plan_dw_px_kernel<3, 3, 2>), grid, dim3(256), 0, s, k);
-          else if (sw == 1) hipLaunchKernelGGL((plan_dw_px_kernel<5, 5, 1>), grid, dim3(256), 0, s, k);
-          else hipLaunchKernelGGL((plan_dw_px_kernel<5, 5, 2>), grid, dim3(256), 0, s, k);
+      // the windowed kernel's offsets are 32-bit, a map's bytes within 2^30
+      const int64_t lim = 1ll << 26;   // float4s
+      if (((kh == 3 && kw == 3) || (kh == 5 && kw == 5)) && (sw == 1 || sw == 2) &&
+          ih * iw * (C / 4) <= lim && P * (C / 4) <= lim && taps * (C / 4) <= lim &&
+          sh < 16 && pt < (1 << 20) && pl_ < (1 << 20)) {
+        return add_launch(pl, d.idx, [k, nb, kh, sw](hipStream_t s) {
+          if (kh == 3 && sw == 1) launch_plan_dw_px<3, 1>(k, (unsigned)nb, s);
+          else if (kh == 3) launch_plan_dw_px<3, 2>(k, (unsigned)nb, s);
+          else if (sw == 1) launch_plan_dw_px<5, 1>(k, (unsigned)nb, s);
+          else launch_plan_dw_px<5, 2>(k, (unsigned)nb, s);
           return launch_check("plan_dw_px_kernel");
         });
       }
@@ -2283,7 +2340,7 @@ int decode(Decoder& d, const qph_plan_dispatch& q, std::vector<PendingHw>& pendi
                      w2[2] == OFF_NONE ? nullptr : d.at(w2[2]), d.at(ex[1]), (int)ih, (int)iw, 4,
                      (int)ex[3], act, act2, ex[7] == 4};
         return add_launch(pl, d.idx, [f, nb](hipStream_t s) {
-          const dim3 grid((unsigned)((f.h * f.w + 255) / 256), 4, (unsigned)nb);
+          const dim3 grid((unsigned)ceil_div((int64_t)f.h * f.w, 64), (unsigned)nb);
           hipLaunchKernelGGL((plan_convt_pair_kernel<24, 24>), grid, dim3(256), 0, s, f);
           return launch_check("plan_convt_pair_kernel");
         });
