@@ -527,6 +527,9 @@ __global__ __launch_bounds__(256) void conv3x3_direct_group_kernel(DirectConvGro
 // spare area) so that every wave issues exactly 4 a chunk and each wait
 // counts exactly the chunks still loading.  The image width is a multiple of
 // 4, so a 16-byte halo group lies wholly inside or wholly outside a row.
+// Other widths (NARROW: the coarse levels of a page whose sides are not
+// multiples of 128) bring the same halo words by 20 one-word loads, 32 loads
+// a chunk in all.
 // Each direct3x3_unit step costs two vector-memory loads per lane; here a
 // step is three LDS reads and two MFMAs.
 
@@ -558,6 +561,7 @@ struct LdsConvGroup {
   DirectConvK k[DIRECT_GROUP_MAX];
   int tiles_x[DIRECT_GROUP_MAX];
   int start[DIRECT_GROUP_MAX + 1];   // start[i] = total for i >= n
+  int narrow[DIRECT_GROUP_MAX];
   int n;
 };
 
@@ -570,7 +574,7 @@ struct LdsConvGroup {
 // read from LDS before its MFMAs (so the reads' latency is paid once a chunk,
 // not once a step), and AK (0 none, 2 ReLU, -1 any kind through act_apply)
 // keeps the epilogue free of the generic activation switch.
-template <int AK, bool ONE, bool CVT = false>
+template <int AK, bool ONE, bool CVT = false, bool NARROW = false>
 __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x, int tile,
                                               float* s0, float* s1, float* s2, float* s3,
                                               int wave, int lane,
@@ -594,11 +598,18 @@ __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x,
   // the 16-byte groups 64 j + lane of the stage (halo groups, then weight
   // groups, then spare ones); the channel / weight-row part of the address
   // is the scalar offset
-  unsigned doff[4];
+  constexpr int PER = NARROW ? 8 : LC_DMA / 4;              // loads per wave per chunk
+  constexpr int HL = NARROW ? LC_HALO / 64 : LC_HALO / 256; // the chunk's halo loads
+  unsigned doff[PER];
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int gi = 64 * (wave + 4 * q) + lane;
-    if (gi < LC_HALO / 4) {
+  for (int q = 0; q < PER; q++) {
+    const int j = wave + 4 * q, gi = 64 * (NARROW ? j - HL + LC_HALO / 256 : j) + lane;
+    if (NARROW && j < HL) {
+      const int wi = 64 * j + lane, cl = wi / (4 * LC_HP), rem = wi - cl * 4 * LC_HP;
+      const int rr = rem / LC_HP, ix = ox0 - 4 + rem - rr * LC_HP, iy = oy0 - 1 + rr;
+      const bool ok = iy >= 0 && iy < p.h && ix >= 0 && ix < p.w;
+      doff[q] = ok ? (unsigned)((cl * HW + iy * p.w + ix) * 4) : OOB;
+    } else if (!NARROW && gi < LC_HALO / 4) {
       const int cl = gi / (4 * LC_HG), rem = gi - cl * 4 * LC_HG;
       const int rr = rem / LC_HG, gc = rem - rr * LC_HG;
       const int iy = oy0 - 1 + rr, ix = ox0 - 4 + 4 * gc;
@@ -626,18 +637,25 @@ __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x,
   const unsigned wstep = __builtin_amdgcn_readfirstlane(LC_WROWS * p.mpad * 4);
   auto issue = [&](int ch, float* st) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
+    for (int q = 0; q < PER; q++) {
       const int j = wave + 4 * q;   // wave-uniform
-      const bool halo = j < LC_HALO / 256;
+      const bool halo = j < HL;
+      // (NARROW: the last spare load repeats the second one's slot)
+      const int at = !NARROW ? 256 * j : halo ? 64 * j : LC_HALO + 256 * min(j - HL, 10);
       const unsigned lds = __builtin_amdgcn_readfirstlane(
-          (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)(st + 256 * j));
+          (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)(st + at));
       const unsigned soff = ch * (halo ? hstep : wstep);
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
-      __asm__ volatile(
-          "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
-          "v"(doff[q]), "s"(halo ? xr : wr), "s"(soff)
-          : "m0");
+      if (NARROW && halo)
+        __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds),
+                         "v"(doff[q]), "s"(xr), "s"(soff)
+                         : "m0");
+      else
+        __asm__ volatile(
+            "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
+            "v"(doff[q]), "s"(halo ? xr : wr), "s"(soff)
+            : "m0");
 #pragma clang diagnostic pop
     }
   };
@@ -702,7 +720,6 @@ __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x,
     boff[s] = cl * 4 * LC_HP + (r + ky) * LC_HP + c + kx + 3;
   }
 
-  constexpr int PER = LC_DMA / 4;   // loads per wave per chunk
   auto stage = [&](auto st) -> float* {
     constexpr int S = decltype(st)::value;
     if constexpr (S == 0) return s0;
@@ -894,7 +911,7 @@ __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x,
     }
 }
 
-template <int AK, int NG>
+template <int AK, int NG, bool NARROW>
 __global__ __launch_bounds__(256) void conv3x3_lds_kernel(LdsConvGroup g) {
   __shared__ __attribute__((aligned(16))) float s0[LC_STAGE], s1[LC_STAGE], s2[LC_STAGE];
   const int lane = threadIdx.x & 63;
@@ -903,12 +920,17 @@ __global__ __launch_bounds__(256) void conv3x3_lds_kernel(LdsConvGroup g) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
   const int t = blockIdx.x;   // < start[DIRECT_GROUP_MAX]: the grid is the total
   if constexpr (NG == 1) {
-    lds_conv_tile<AK, false>(g.k[0], g.tiles_x[0], t, s0, s1, s2, nullptr, wave, lane);
+    lds_conv_tile<AK, false, false, NARROW>(g.k[0], g.tiles_x[0], t, s0, s1, s2, nullptr, wave,
+                                            lane);
   } else {
     // the member conv, without branches: start[] is non-decreasing
     const int i = (t >= g.start[1]) + (t >= g.start[2]) + (t >= g.start[3]);
-    lds_conv_tile<AK, false>(g.k[i], g.tiles_x[i], t - g.start[i], s0, s1, s2, nullptr, wave,
-                             lane);
+    if (NARROW && g.narrow[i])
+      lds_conv_tile<AK, false, false, true>(g.k[i], g.tiles_x[i], t - g.start[i], s0, s1, s2,
+                                            nullptr, wave, lane);
+    else
+      lds_conv_tile<AK, false>(g.k[i], g.tiles_x[i], t - g.start[i], s0, s1, s2, nullptr, wave,
+                               lane);
   }
 }
 
@@ -970,16 +992,49 @@ bool direct3x3_eligible(const ConvArgs& a) {
 static bool lds3x3_eligible(const ConvArgs& a) {
   return direct3x3_eligible(a) && a.sh == 1 && a.sw == 1 && a.ph == 1 && a.pw == 1 &&
          a.m <= 32 && a.c % LC_CC == 0 && a.c > 0 && mpad_of(a.m) == 32 &&
-         a.c * a.h * a.w * 4 < (int64_t)0x80000000 && a.w % 4 == 0 &&
-         (uintptr_t)a.x % 16 == 0;
+         a.c * a.h * a.w * 4 < (int64_t)0x80000000;
+}
+
+// whether the halo's 16-byte loads are aligned and whole
+static bool lds3x3_wide(const ConvArgs& a) { return a.w % 4 == 0 && (uintptr_t)a.x % 16 == 0; }
+
+template <int AK>
+static void launch_lds_ring(const LdsConvGroup& g, dim3 grid, bool narrow, hipStream_t s) {
+  if (g.n == 1 && narrow)
+    hipLaunchKernelGGL((conv3x3_lds_kernel<AK, 1, true>), grid, dim3(256), 0, s, g);
+  else if (g.n == 1)
+    hipLaunchKernelGGL((conv3x3_lds_kernel<AK, 1, false>), grid, dim3(256), 0, s, g);
+  else if (narrow)
+    hipLaunchKernelGGL((conv3x3_lds_kernel<AK, 4, true>), grid, dim3(256), 0, s, g);
+  else
+    hipLaunchKernelGGL((conv3x3_lds_kernel<AK, 4, false>), grid, dim3(256), 0, s, g);
+}
+
+// Whether the LDS kernel takes the convs of one launch.  With the halo by
+// one-word loads it needs enough tiles to fill the CUs: 96 -> 24 channels,
+// direct against LDS: 80x81 (120 tiles) 11.1 and 13.5 us, 100x101 (200) 15.7
+// and 13.6, 160x161 (480) 25.6 and 21.6; 32 -> 32 channels the same way round.
+#define LDS_NARROW_TILES 160
+static bool lds3x3_pays(const ConvArgs* a, int n) {
+  int64_t tiles = 0;
+  bool narrow = false;
+  for (int i = 0; i < n; i++) {
+    if (!lds3x3_eligible(a[i])) return false;
+    narrow = narrow || !lds3x3_wide(a[i]);
+    tiles += (int64_t)ceil_div(a[i].ow, 32) * ceil_div(a[i].oh, 2) * a[i].n;
+  }
+  return !narrow || tiles >= LDS_NARROW_TILES;
 }
 
 static int launch_lds3x3(const ConvArgs* a, int n, hipStream_t s) {
   LdsConvGroup g{};
   g.n = n;
   int64_t total = 0;
+  bool narrow = false;
   for (int i = 0; i < n; i++) {
     direct_params(a[i], a[i].wk, g.k[i]);
+    g.narrow[i] = !lds3x3_wide(a[i]);
+    narrow = narrow || g.narrow[i];
     g.tiles_x[i] = (int)ceil_div(a[i].ow, 32);
     g.start[i] = (int)total;
     total += (int64_t)g.tiles_x[i] * ceil_div(a[i].oh, 2) * a[i].n;
@@ -990,7 +1045,7 @@ static int launch_lds3x3(const ConvArgs* a, int n, hipStream_t s) {
   for (int i = 1; i < n; i++)
     if (a[i].act.kind != kind) kind = -1;
   const dim3 grid((unsigned)total);
-  if (n == 1 && a[0].c == 32 && (kind == 0 || kind == 2) && !a[0].res && a[0].y_up == 1 &&
+  if (n == 1 && !narrow && a[0].c == 32 && (kind == 0 || kind == 2) && !a[0].res && a[0].y_up == 1 &&
       a[0].y_ctotal < (1ll << 31) && a[0].y_coff < (1ll << 31)) {
     const DirectConvK& k = g.k[0];
     if (kind == 0)
@@ -1001,21 +1056,12 @@ static int launch_lds3x3(const ConvArgs* a, int n, hipStream_t s) {
                          k.h, k.w, k.m, g.tiles_x[0], (int)k.y_ctotal, (int)k.y_coff);
     return launch_check("conv3x3_lds32_kernel");
   }
-  if (n == 1) {
-    if (kind == 0)
-      hipLaunchKernelGGL((conv3x3_lds_kernel<0, 1>), grid, dim3(256), 0, s, g);
-    else if (kind == 2)
-      hipLaunchKernelGGL((conv3x3_lds_kernel<2, 1>), grid, dim3(256), 0, s, g);
-    else
-      hipLaunchKernelGGL((conv3x3_lds_kernel<-1, 1>), grid, dim3(256), 0, s, g);
-  } else {
-    if (kind == 0)
-      hipLaunchKernelGGL((conv3x3_lds_kernel<0, 4>), grid, dim3(256), 0, s, g);
-    else if (kind == 2)
-      hipLaunchKernelGGL((conv3x3_lds_kernel<2, 4>), grid, dim3(256), 0, s, g);
-    else
-      hipLaunchKernelGGL((conv3x3_lds_kernel<-1, 4>), grid, dim3(256), 0, s, g);
-  }
+  if (kind == 0)
+    launch_lds_ring<0>(g, grid, narrow, s);
+  else if (kind == 2)
+    launch_lds_ring<2>(g, grid, narrow, s);
+  else
+    launch_lds_ring<-1>(g, grid, narrow, s);
   return launch_check("conv3x3_lds_kernel");
 }
 
@@ -1024,7 +1070,7 @@ static int launch_lds3x3(const ConvArgs* a, int n, hipStream_t s) {
 // lds_conv_tile takes, stored plainly (no residual, slot or upsample), ReLU
 // or no activation.
 bool conv3x3_convt_eligible(const ConvArgs& a) {
-  return lds3x3_eligible(a) && a.m == CV_C && !a.res && a.y_up == 1 &&
+  return lds3x3_eligible(a) && lds3x3_wide(a) && a.m == CV_C && !a.res && a.y_up == 1 &&
          (a.y_ctotal == 0 || a.y_ctotal == a.m) && a.y_coff == 0 &&
          (a.act.kind == 0 || a.act.kind == 2) && a.n * 16 * a.oh * a.ow < (1ll << 31);
 }
@@ -1051,8 +1097,8 @@ int launch_conv3x3_convt(const ConvArgs& a, const float* w1, const float* w2, fl
 int launch_dense_conv_group(const ConvArgs* a, int n, hipStream_t s) {
   if (n < 1 || n > DIRECT_GROUP_MAX) return fail(QPH_EINVAL, "conv group: 1 to 4 convs");
   bool lds = true;
-  for (int i = 0; i < n; i++) lds = lds && a[i].wk && lds3x3_eligible(a[i]);
-  if (lds) return launch_lds3x3(a, n, s);
+  for (int i = 0; i < n; i++) lds = lds && a[i].wk;
+  if (lds && lds3x3_pays(a, n)) return launch_lds3x3(a, n, s);
   DirectConvGroup g{};
   g.n = n;
   int64_t total = 0;
@@ -1076,7 +1122,7 @@ int launch_dense_conv_group(const ConvArgs* a, int n, hipStream_t s) {
 // Launches the direct kernel for a 3x3 conv, choosing the per-wave tile so
 // that the launch has enough waves to hide load latency.
 static int launch_direct3x3(const ConvArgs& a, const float* wk, hipStream_t s) {
-  if (lds3x3_eligible(a)) {
+  if (lds3x3_pays(&a, 1)) {
     ConvArgs b = a;
     b.wk = wk;
     return launch_lds3x3(&b, 1, s);

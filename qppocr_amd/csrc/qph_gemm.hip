@@ -333,16 +333,20 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(GemmArgs g) {
 // slabs of 16 through an NST-stage LDS ring filled by 16-byte buffer->LDS
 // loads: one for the X slab (16 rows x 16 columns) and MBW for the W slab
 // (16 k of each row, its four 16-byte chunks rotated by row % 4 so that the
-// A reads of one step spread over the banks).  The wave waits only on its own
+// A reads of one step spread over the banks).  Where the X rows are not
+// 16-byte aligned or N is not a multiple of 4 (!WIDE: maps of odd sides, as
+// the coarse levels of a 160x416 crop), the X slab comes by four one-word
+// loads of the same slots.  The wave waits only on its own
 // loads: no workgroup barrier.  Bias and residual terms are loaded before
 // the first slab, so the slab waits, which count loads in issue order, never
 // wait for them.  The loads are inline asm, so the compiler adds no waits
 // of its own for the stages.
-template <int MBW, int NST>
+template <int MBW, int NST, bool WIDE>
 __device__ __forceinline__ void pw_tile(const GemmArgs& g, int mgroups, int blk, int64_t bt,
                                         float* pw_lds) {
   constexpr int STAGE = 256 * (1 + MBW);   // floats: X slab, then W slab
-  constexpr int PER = 1 + MBW;             // loads per slab
+  constexpr int XL = WIDE ? 1 : 4;         // X loads per slab
+  constexpr int PER = XL + MBW;            // loads per slab
   if (g.rn && *g.rn != 0 && bt >= (int64_t)*g.rn * g.rn_per) return;   // past the real batch
   const int lane = threadIdx.x;
   const int l16 = lane & 15, lg = lane >> 4;
@@ -374,8 +378,10 @@ __device__ __forceinline__ void pw_tile(const GemmArgs& g, int mgroups, int blk,
       (void*)Bb, 0, (int)(g.k * g.ldb * 4), 0x00020000);
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)Ab, 0, (int)(M * g.lda * 4), 0x00020000);
-  const int xrow = lane >> 2, xc = lane & 3;
-  const unsigned xoff = (n0 + 4 * xc < N) ? (unsigned)((xrow * g.ldb + n0 + 4 * xc) * 4) : OOB;
+  // X slot: WIDE row lane / 4, columns 4 (lane % 4) .. + 3; else row
+  // 4 q + lane / 16 of load q, column lane % 16
+  const int xrow = WIDE ? lane >> 2 : lg, xc = WIDE ? 4 * (lane & 3) : l16;
+  const unsigned xoff = (n0 + xc < N) ? (unsigned)((xrow * g.ldb + n0 + xc) * 4) : OOB;
   unsigned woff[MBW];
 #pragma unroll
   for (int q = 0; q < MBW; q++) {
@@ -391,9 +397,18 @@ __device__ __forceinline__ void pw_tile(const GemmArgs& g, int mgroups, int blk,
     const unsigned sx = (unsigned)q * xstep, sw = (unsigned)q * 64u;
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
-    __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lx),
-                     "v"(xoff), "s"(xr), "s"(sx)
-                     : "m0");
+    if constexpr (WIDE) {
+      __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lx),
+                       "v"(xoff), "s"(xr), "s"(sx)
+                       : "m0");
+    } else {
+#pragma unroll
+      for (int x = 0; x < XL; x++)
+        __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(
+                             lx + 256u * x),
+                         "v"(xoff), "s"(xr), "s"(sx + x * (xstep >> 2))
+                         : "m0");
+    }
 #pragma unroll
     for (int w = 0; w < MBW; w++)
       __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(
@@ -474,10 +489,10 @@ __device__ __forceinline__ void pw_tile(const GemmArgs& g, int mgroups, int blk,
     }
 }
 
-template <int MBW, int NST>
+template <int MBW, int NST, bool WIDE>
 __global__ __launch_bounds__(64) void gemm_pw_kernel(GemmArgs g, int mgroups) {
   extern __shared__ float pw_lds[];
-  pw_tile<MBW, NST>(g, mgroups, blockIdx.x, blockIdx.z, pw_lds);
+  pw_tile<MBW, NST, WIDE>(g, mgroups, blockIdx.x, blockIdx.z, pw_lds);
 }
 
 // Up to three independent pointwise GEMMs in one launch, one 16-row block a
@@ -488,28 +503,44 @@ struct PwGroup {
   GemmArgs g[3];
   int mgroups[3];
   int start[3];
+  int wide[3];
 };
 
 template <int NST>
 __global__ __launch_bounds__(64) void gemm_pw_group_kernel(PwGroup p) {
   extern __shared__ float pw_lds[];
   const int b = blockIdx.x;
-  if (b >= p.start[2])
-    pw_tile<1, NST>(p.g[2], p.mgroups[2], b - p.start[2], blockIdx.z, pw_lds);
-  else if (b >= p.start[1])
-    pw_tile<1, NST>(p.g[1], p.mgroups[1], b - p.start[1], blockIdx.z, pw_lds);
-  else
-    pw_tile<1, NST>(p.g[0], p.mgroups[0], b, blockIdx.z, pw_lds);
+#define PW_MEMBER(I)                                                                          \
+  if (p.wide[I])                                                                              \
+    pw_tile<1, NST, true>(p.g[I], p.mgroups[I], b - p.start[I], blockIdx.z, pw_lds);          \
+  else                                                                                        \
+    pw_tile<1, NST, false>(p.g[I], p.mgroups[I], b - p.start[I], blockIdx.z, pw_lds)
+  if (b >= p.start[2]) {
+    PW_MEMBER(2);
+  } else if (b >= p.start[1]) {
+    PW_MEMBER(1);
+  } else {
+    PW_MEMBER(0);
+  }
+#undef PW_MEMBER
 }
 
-// The pointwise kernel takes K a multiple of 16, M <= 128, 16-byte aligned
-// rows of both operands, N a multiple of 4 and offsets within 31 bits.
+// The pointwise kernel takes K a multiple of 16, 16-byte aligned rows of A
+// and offsets within 31 bits, up to 512 output channels (the skinny kernel's
+// 32 x 32 tiles measured slower over that range: 96x1089x128 7.9 against 5.2
+// us, 96x25921x64 25.5 against 17.9, 32 maps of 256x36x256 10.9 against 7.8,
+// 256x10000x256 34.1 against 32.1; past it no net here has a conv).
+#define PW_MAX_M 512
 static bool pw_eligible(const GemmArgs& g) {
   return !g.trans_out && g.part == nullptr && g.bias_mode != 2 && g.k % 16 == 0 &&
-         g.k >= 16 && g.m <= 128 && g.n % 4 == 0 && g.ldb % 4 == 0 && g.lda % 4 == 0 &&
-         g.a_batch % 4 == 0 && g.b_batch % 4 == 0 && (uintptr_t)g.a % 16 == 0 &&
-         (uintptr_t)g.b % 16 == 0 && g.k * g.ldb * 4 < (1ll << 31) &&
+         g.k >= 16 && g.m <= PW_MAX_M && g.lda % 4 == 0 && g.a_batch % 4 == 0 &&
+         (uintptr_t)g.a % 16 == 0 && g.k * g.ldb * 4 < (1ll << 31) &&
          g.m * g.lda * 4 < (1ll << 31) && g.ldb >= g.n && g.lda >= g.k;
+}
+
+// whether the X slab's 16-byte loads are aligned and whole
+static bool pw_wide(const GemmArgs& g) {
+  return g.n % 4 == 0 && g.ldb % 4 == 0 && g.b_batch % 4 == 0 && (uintptr_t)g.b % 16 == 0;
 }
 
 bool pw_group_eligible(const GemmArgs& g) {
@@ -528,6 +559,7 @@ int launch_pw_group(const GemmArgs* g, int n, hipStream_t s) {
     p.g[i] = g[i];
     p.mgroups[i] = (int)ceil_div(g[i].m, 16);
     p.start[i] = (int)total;
+    p.wide[i] = pw_wide(g[i]);
     total += ceil_div(g[i].n, 16) * p.mgroups[i];
     deep = deep || g[i].k > 32;
   }
@@ -590,40 +622,49 @@ int launch_fpn_topdown(const float* t4, const float* in5, const float* t3, float
   return launch_check("fpn_topdown_kernel");
 }
 
-template <int MBW>
+template <int MBW, bool WIDE>
 static void launch_pw_m(const GemmArgs& g, int mgroups, dim3 grid, bool deep, hipStream_t s) {
   const size_t lds = (size_t)(deep ? 4 : 2) * 256 * (1 + MBW) * 4;
   if (deep)
-    hipLaunchKernelGGL((gemm_pw_kernel<MBW, 4>), grid, dim3(64), lds, s, g, mgroups);
+    hipLaunchKernelGGL((gemm_pw_kernel<MBW, 4, WIDE>), grid, dim3(64), lds, s, g, mgroups);
   else
-    hipLaunchKernelGGL((gemm_pw_kernel<MBW, 2>), grid, dim3(64), lds, s, g, mgroups);
+    hipLaunchKernelGGL((gemm_pw_kernel<MBW, 2, WIDE>), grid, dim3(64), lds, s, g, mgroups);
+}
+
+template <bool WIDE>
+static void launch_pw_w(int mbw, const GemmArgs& g, int mgroups, dim3 grid, hipStream_t s) {
+  const bool deep = g.k > 32;
+  switch (mbw) {
+    case 1: launch_pw_m<1, WIDE>(g, mgroups, grid, deep, s); break;
+    case 2: launch_pw_m<2, WIDE>(g, mgroups, grid, deep, s); break;
+    case 3: launch_pw_m<3, WIDE>(g, mgroups, grid, deep, s); break;
+    case 4: launch_pw_m<4, WIDE>(g, mgroups, grid, deep, s); break;
+    case 5: launch_pw_m<5, WIDE>(g, mgroups, grid, deep, s); break;
+    case 6: launch_pw_m<6, WIDE>(g, mgroups, grid, deep, s); break;
+    case 7: launch_pw_m<7, WIDE>(g, mgroups, grid, deep, s); break;
+    default: launch_pw_m<8, WIDE>(g, mgroups, grid, deep, s); break;
+  }
 }
 
 static int launch_pw(const GemmArgs& g, hipStream_t s) {
   const int mb = (int)ceil_div(g.m, 16);
   const int64_t pgroups = ceil_div(g.n, 16);
-  // blocks per wave: the largest divisor of mb that still leaves >= 2048
-  // waves (else 1): more blocks share one X slab, fewer spread the chains
+  // blocks per wave: the most, up to 8, that still leave >= 2048 waves (else
+  // 1) and at most one block in nine past M: more blocks share one X slab,
+  // fewer spread the chains
   int mbw = 1;
-  for (int c = mb; c >= 1; c--)
-    if (mb % c == 0 && pgroups * (mb / c) * g.batch >= 2048) {
+  for (int c = mb < 8 ? mb : 8; c >= 1; c--)
+    if ((ceil_div(mb, c) * c - mb) * 8 <= mb && pgroups * ceil_div(mb, c) * g.batch >= 2048) {
       mbw = c;
       break;
     }
-  const int mgroups = mb / mbw;
+  const int mgroups = (int)ceil_div(mb, mbw);
   if (pgroups * mgroups >= (1ll << 31)) return fail(QPH_EUNSUPPORTED, "gemm: grid too large");
   dim3 grid((unsigned)(pgroups * mgroups), 1, (unsigned)g.batch);
-  const bool deep = g.k > 32;
-  switch (mbw) {
-    case 1: launch_pw_m<1>(g, mgroups, grid, deep, s); break;
-    case 2: launch_pw_m<2>(g, mgroups, grid, deep, s); break;
-    case 3: launch_pw_m<3>(g, mgroups, grid, deep, s); break;
-    case 4: launch_pw_m<4>(g, mgroups, grid, deep, s); break;
-    case 5: launch_pw_m<5>(g, mgroups, grid, deep, s); break;
-    case 6: launch_pw_m<6>(g, mgroups, grid, deep, s); break;
-    case 7: launch_pw_m<7>(g, mgroups, grid, deep, s); break;
-    default: launch_pw_m<8>(g, mgroups, grid, deep, s); break;
-  }
+  if (pw_wide(g))
+    launch_pw_w<true>(mbw, g, mgroups, grid, s);
+  else
+    launch_pw_w<false>(mbw, g, mgroups, grid, s);
   return launch_check("gemm_pw_kernel");
 }
 
