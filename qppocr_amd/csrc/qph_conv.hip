@@ -561,7 +561,6 @@ struct LdsConvGroup {
   DirectConvK k[DIRECT_GROUP_MAX];
   int tiles_x[DIRECT_GROUP_MAX];
   int start[DIRECT_GROUP_MAX + 1];   // start[i] = total for i >= n
-  int narrow[DIRECT_GROUP_MAX];
   int n;
 };
 
@@ -574,6 +573,68 @@ struct LdsConvGroup {
 // read from LDS before its MFMAs (so the reads' latency is paid once a chunk,
 // not once a step), and AK (0 none, 2 ReLU, -1 any kind through act_apply)
 // keeps the epilogue free of the generic activation switch.
+// The conv-transpose pair over NJ tiles of 16 conv outputs of a row, columns
+// pox + 16 j, that this wave wrote to hh ([pixel][CV_HP]): the A operands and
+// w2 through fb, then the products, the second chain and the sigmoid.
+template <int NJ>
+__device__ __forceinline__ void convt_finish(const DirectConvK& p, const ConvtEpi& cv,
+                                             const float* hh, float* fb, const float* w1r,
+                                             float w2r, int wave, int lane, int img, int poy,
+                                             int pox0) {
+  const int l16 = lane & 15, lg = lane >> 4;
+  // A operands in MFMA order [mt][s][lane]: lane g 16 + i of step s, tile mt
+  // holds w1[ci = 4 s + g][co = 4 mt + (i & 3)][q = i >> 2]
+  float* sa = fb;
+  float* sw2 = fb + 4 * CV_C * CV_C;  // [co][q2]
+  {
+    const int tid = wave * 64 + lane;
+#pragma unroll
+    for (int j = 0; j < 9; j++) {
+      const int i = tid + 256 * j;   // (ci * 24 + co) * 4 + q
+      const int ci = i / (4 * CV_C), co = (i >> 2) % CV_C, q = i & 3;
+      sa[((co >> 2) * (CV_C / 4) + (ci >> 2)) * 64 + (ci & 3) * 16 + q * 4 + (co & 3)] = w1r[j];
+    }
+    if (tid < 4 * CV_C) sw2[tid] = w2r;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    // every lane takes part in the products (an idle lane's A row would be
+    // lost to every pixel); only the stores are per pixel
+    float bx[CV_C / 4];
+#pragma unroll
+    for (int s = 0; s < CV_C / 4; s++) bx[s] = hh[(16 * j + l16) * CV_HP + 4 * s + lg];
+    f32x4 mid[CV_C / 4];
+#pragma unroll
+    for (int mt = 0; mt < CV_C / 4; mt++) {
+      mid[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < CV_C / 4; s++)
+        mid[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[(mt * (CV_C / 4) + s) * 64 + lane], bx[s],
+                                                       mid[mt], 0, 0, 0);
+    }
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int co = 0; co < CV_C; co++) {
+      const f32x4 wv = *(const f32x4*)(sw2 + co * 4);
+      const float mv = mid[co >> 2][co & 3];
+      o[0] = __builtin_fmaf(mv, wv[0], o[0]);
+      o[1] = __builtin_fmaf(mv, wv[1], o[1]);
+      o[2] = __builtin_fmaf(mv, wv[2], o[2]);
+      o[3] = __builtin_fmaf(mv, wv[3], o[3]);
+    }
+    const int pox = pox0 + 16 * j;
+    if (poy >= p.oh || pox >= p.ow) continue;
+    const int ky = lg >> 1, kx = lg & 1;
+    const int64_t ow4 = 4 * (int64_t)p.ow;
+    float* yo = cv.y + ((int64_t)img * 4 * p.oh + 4 * poy + 2 * ky) * ow4 + 4 * pox + 2 * kx;
+    yo[0] = sigmoid1(o[0]);
+    yo[1] = sigmoid1(o[1]);
+    yo[ow4] = sigmoid1(o[2]);
+    yo[ow4 + 1] = sigmoid1(o[3]);
+  }
+}
+
 template <int AK, bool ONE, bool CVT = false, bool NARROW = false>
 __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x, int tile,
                                               float* s0, float* s1, float* s2, float* s3,
@@ -831,53 +892,7 @@ __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x,
           xv = act_apply(xv, p.act);
         if (co < CV_C) hh[l16 * CV_HP + co] = xv;
       }
-    // A operands in MFMA order [mt][s][lane]: lane g 16 + i of step s, tile mt
-    // holds w1[ci = 4 s + g][co = 4 mt + (i & 3)][q = i >> 2]
-    float* sa = fb;
-    float* sw2 = fb + 4 * CV_C * CV_C;  // [co][q2]
-    {
-      const int tid = wave * 64 + lane;
-#pragma unroll
-      for (int j = 0; j < 9; j++) {
-        const int i = tid + 256 * j;   // (ci * 24 + co) * 4 + q
-        const int ci = i / (4 * CV_C), co = (i >> 2) % CV_C, q = i & 3;
-        sa[((co >> 2) * (CV_C / 4) + (ci >> 2)) * 64 + (ci & 3) * 16 + q * 4 + (co & 3)] = w1r[j];
-      }
-      if (tid < 4 * CV_C) sw2[tid] = w2r;
-    }
-    __syncthreads();
-    // every lane takes part in the products (an idle lane's A row would be
-    // lost to every pixel); only the stores are per pixel
-    float bx[CV_C / 4];
-#pragma unroll
-    for (int s = 0; s < CV_C / 4; s++) bx[s] = hh[l16 * CV_HP + 4 * s + lg];
-    f32x4 mid[CV_C / 4];
-#pragma unroll
-    for (int mt = 0; mt < CV_C / 4; mt++) {
-      mid[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int s = 0; s < CV_C / 4; s++)
-        mid[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[(mt * (CV_C / 4) + s) * 64 + lane], bx[s],
-                                                       mid[mt], 0, 0, 0);
-    }
-    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int co = 0; co < CV_C; co++) {
-      const f32x4 wv = *(const f32x4*)(sw2 + co * 4);
-      const float mv = mid[co >> 2][co & 3];
-      o[0] = __builtin_fmaf(mv, wv[0], o[0]);
-      o[1] = __builtin_fmaf(mv, wv[1], o[1]);
-      o[2] = __builtin_fmaf(mv, wv[2], o[2]);
-      o[3] = __builtin_fmaf(mv, wv[3], o[3]);
-    }
-    if (!pval) return;
-    const int ky = lg >> 1, kx = lg & 1;
-    const int64_t ow4 = 4 * (int64_t)p.ow;
-    float* yo = cv.y + ((int64_t)img * 4 * p.oh + 4 * poy + 2 * ky) * ow4 + 4 * pox + 2 * kx;
-    yo[0] = sigmoid1(o[0]);
-    yo[1] = sigmoid1(o[1]);
-    yo[ow4] = sigmoid1(o[2]);
-    yo[ow4 + 1] = sigmoid1(o[3]);
+    convt_finish<1>(p, cv, hh, fb, w1r, w2r, wave, lane, img, poy, pox);
     return;
   }
   // epilogue as in direct3x3_unit; every residual term is read before the
@@ -925,12 +940,8 @@ __global__ __launch_bounds__(256) void conv3x3_lds_kernel(LdsConvGroup g) {
   } else {
     // the member conv, without branches: start[] is non-decreasing
     const int i = (t >= g.start[1]) + (t >= g.start[2]) + (t >= g.start[3]);
-    if (NARROW && g.narrow[i])
-      lds_conv_tile<AK, false, false, true>(g.k[i], g.tiles_x[i], t - g.start[i], s0, s1, s2,
+    lds_conv_tile<AK, false, false, NARROW>(g.k[i], g.tiles_x[i], t - g.start[i], s0, s1, s2,
                                             nullptr, wave, lane);
-    else
-      lds_conv_tile<AK, false>(g.k[i], g.tiles_x[i], t - g.start[i], s0, s1, s2, nullptr, wave,
-                               lane);
   }
 }
 
@@ -945,6 +956,294 @@ __global__ __launch_bounds__(256) void conv3x3_lds_convt_kernel(DirectConvK k, i
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
   lds_conv_tile<AK, false, true>(k, tiles_x, blockIdx.x, s0, s1, s2, nullptr, wave, lane, cv);
+}
+
+// ------------------------------------ 17 to 24 output channels, large maps
+//
+// The det neck and head have 24 output channels: in lds_conv_tile the second
+// 16-row MFMA of every step does half its work for padding, and a tile of 64
+// pixels reloads all 9 KB of a chunk's weights.  Here a workgroup takes 4 rows
+// of 32 pixels, a wave one row: channels 0-15 as two 16x16x4 chains, channels
+// 16-23 as one chain of 4x4x1 MFMAs, whose 16 blocks are 2 channel quads by 8
+// pixel quads (lane: channel quad lane / 32, pixel lane % 32).  One register
+// holds the tail's A operand of 8 k (block 8 q + e: channels 16 + 4 q .. + 3 at
+// k + e), picked by the A block broadcast; one holds its B operand of two k
+// (lanes 0-31 and 32-63), picked by the B lane-half broadcast.  A step of 4 k
+// and 32 pixels takes 49 ns of a SIMD's matrix unit against 62, reads 5.5
+// words a lane from LDS against 6, and half the weight bytes from L2.  The
+// chains are the same fma chains in the same k order.
+//
+// A stage holds 8 channels' halo (6 rows of 40 columns, LT_HALO words padded
+// to whole loads), then the 72 weight rows' first 24 columns, then spare
+// words; NARROW as in lds_conv_tile.  Two stages: with three workgroups on a
+// CU the next chunk has their combined time to arrive.  Neck and head of a
+// 1536x1536 page 112 -> 103 and 90 -> 82 us, 960x960 57 -> 51 and 42 -> 36
+// (86 and 70 on the large page without any operand reads or loads: the rest is
+// the matrix units, the workgroups' start and their stores).
+#define LT_HALO 1920                        // 8 x 6 x 40
+#define LT_HALO_PAD 2048
+#define LT_WC 24                            // weight columns kept
+#define LT_W (LC_WROWS * LT_WC)             // 1728 words
+#define LT_STAGE 4096
+#define LT_PLANE (6 * LC_HP)
+
+template <int E>   // the tail's product of the e-th k of an 8-k block
+__device__ __forceinline__ f32x4 tail_mma(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 3, E, 1 + (E & 1));
+}
+
+template <int AK, bool CVT, bool NARROW>
+__device__ __forceinline__ void tall_conv_tile(const DirectConvK& p, int tiles_x, int tile,
+                                               float* s0, float* s1, int wave, int lane,
+                                               const ConvtEpi& cv = ConvtEpi{}) {
+  __asm__ volatile("" ::"s"(p.x), "s"(p.wk), "s"(p.c), "s"(p.h), "s"(p.w), "s"(p.oh),
+                   "s"(p.ow), "s"(p.mpad), "s"(tiles_x), "s"(tile));
+  const int l16 = lane & 15, lg = lane >> 4, l32 = lane & 31, lh = lane >> 5;
+  const int per_img = tiles_x * ((p.oh + 3) / 4);
+  const int img = tile / per_img, rem = tile - img * per_img;
+  const int oy0 = (rem / tiles_x) * 4, ox0 = (rem % tiles_x) * 32;
+  const int HW = p.h * p.w;
+  const unsigned OOB = 0x80000000u;
+  const int poy = oy0 + wave;
+
+  // load j = wave + 4 q: 16-byte groups (NARROW: words for the halo)
+  constexpr int HL = NARROW ? LT_HALO / 64 : LT_HALO_PAD / 256;   // halo loads: 30 or 8
+  constexpr int PER = NARROW ? 10 : 4;
+  unsigned doff[PER];
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    const int j = wave + 4 * q;
+    doff[q] = OOB;
+    if (j < HL) {
+      const int wi = (NARROW ? 1 : 4) * (64 * j + lane);   // word of the halo
+      const int cl = wi / LT_PLANE, rm = wi - cl * LT_PLANE;
+      const int rr = rm / LC_HP, ix = ox0 - 4 + rm - rr * LC_HP, iy = oy0 - 1 + rr;
+      if (wi < LT_HALO && iy >= 0 && iy < p.h && ix >= 0 && ix < p.w)
+        doff[q] = (unsigned)((cl * HW + iy * p.w + ix) * 4);
+    } else {
+      const int wg = 64 * (j - HL) + lane, kr = wg / (LT_WC / 4), cg = wg - kr * (LT_WC / 4);
+      if (kr < LC_WROWS) doff[q] = (unsigned)((kr * p.mpad + 4 * cg) * 4);
+    }
+  }
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.x + (int64_t)img * p.c * HW), 0, p.c * HW * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.wk, 0, p.c * 9 * p.mpad * 4, 0x00020000);
+  const unsigned hstep = __builtin_amdgcn_readfirstlane(LC_CC * HW * 4);
+  const unsigned wstep = __builtin_amdgcn_readfirstlane(LC_WROWS * p.mpad * 4);
+  auto issue = [&](int ch, float* st) {
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      const int j = wave + 4 * q;   // wave-uniform
+      const bool halo = j < HL;
+      // weight loads 0-6 of 7; loads past the stage repeat its last slot
+      const int at = halo ? (NARROW ? 64 : 256) * j : LT_HALO_PAD + 256 * min(j - HL, 7);
+      const unsigned lds = __builtin_amdgcn_readfirstlane(
+          (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)(st + at));
+      const unsigned soff = ch * (halo ? hstep : wstep);
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
+      if (NARROW && halo)
+        __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds),
+                         "v"(doff[q]), "s"(xr), "s"(soff)
+                         : "m0");
+      else
+        __asm__ volatile(
+            "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
+            "v"(doff[q]), "s"(halo ? xr : wr), "s"(soff)
+            : "m0");
+#pragma clang diagnostic pop
+    }
+  };
+  // bias terms, as in lds_conv_tile: [0..3] channels 4 lg + v, [4..7] channels
+  // 16 + 4 lh + v
+  float bld[8];
+#pragma unroll
+  for (int v = 0; v < 8; v++) {
+    const int co = v < 4 ? 4 * lg + v : 12 + 4 * lh + v;
+    bld[v] = (p.bias && co < p.m) ? p.bias[co] : 0.0f;
+  }
+  float w1r[CVT ? 9 : 1], w2r = 0.0f;
+  if constexpr (CVT) {
+    const int tid = wave * 64 + lane;
+#pragma unroll
+    for (int j = 0; j < 9; j++) w1r[j] = cv.w1[tid + 256 * j];
+    if (tid < 4 * CV_C) w2r = cv.w2[tid];
+  }
+  __asm__ volatile("" ::: "memory");
+  const int nch = p.c / LC_CC;
+  issue(0, s0);
+  __asm__ volatile("" : "+v"(bld[0]), "+v"(bld[1]), "+v"(bld[2]), "+v"(bld[3]), "+v"(bld[4]),
+                   "+v"(bld[5]), "+v"(bld[6]), "+v"(bld[7])::"memory");
+  // the tile's columns are one 32-column panel of the output row
+  const bool tail_panel = (p.ow - ox0) < 32;
+  const int mtail = p.m - p.m % 4;
+  float bterm[8];
+  f32x4 acc[2], tl;   // channels 0-15 of the two 16-pixel tiles, channels 16-23
+#pragma unroll
+  for (int v = 0; v < 8; v++) {
+    const int co = v < 4 ? 4 * lg + v : 12 + 4 * lh + v;
+    const bool seeded = p.bias && tail_panel && co >= mtail;
+    bterm[v] = (p.bias && !seeded) ? bld[v] : -0.0f;
+    const float s = seeded ? bld[v] : 0.0f;
+    if (v < 4) {
+      acc[0][v] = s;
+      acc[1][v] = s;
+    } else {
+      tl[v - 4] = s;
+    }
+  }
+
+  // operand offsets: k = 4 s + lg (period 9 in s: 4 channels) and k = 2 u + lh
+  // (period 9 in u: 2 channels)
+  auto word = [&](int k, int c) {
+    const int cl = k / 9, tap = k - 9 * cl, ky = tap / 3, kx = tap - 3 * ky;
+    return cl * LT_PLANE + (wave + ky) * LC_HP + c + kx + 3;
+  };
+  int bo16[9], bo4[9];
+#pragma unroll
+  for (int i = 0; i < 9; i++) {
+    bo16[i] = word(4 * i + lg, l16);
+    bo4[i] = word(2 * i + lh, l32);
+  }
+  const int ao16 = lg * LT_WC + l16;
+  const int ao4 = ((lane >> 2) & 7) * LT_WC + 16 + 4 * lh + (lane & 3);
+  constexpr int NB = LC_WROWS / 8;   // 8-k blocks
+  auto mma = [&](const float* st) {
+    const float* wst = st + LT_HALO_PAD;
+    float a16[NB][2], b16[NB][2][2], a4[NB], b4[NB][4];
+    auto read = [&](int b) {
+      a4[b] = wst[ao4 + 8 * b * LT_WC];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int s = 2 * b + h;
+        a16[b][h] = wst[ao16 + 4 * s * LT_WC];
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          b16[b][h][j] = st[bo16[s % 9] + (s / 9) * 4 * LT_PLANE + 16 * j];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const int u = 2 * s + i;
+          b4[b][2 * h + i] = st[bo4[u % 9] + (u / 9) * 2 * LT_PLANE];
+        }
+      }
+    };
+    // a block's operand reads run one block ahead of its 12 MFMAs
+    read(0);
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      if (b + 1 < NB) read(b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      // in this order: left alone, the tail's dependent products end up one
+      // after another
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a16[b][0], b16[b][0][0], acc[0], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      tl = tail_mma<0>(a4[b], b4[b][0], tl);
+      tl = tail_mma<1>(a4[b], b4[b][0], tl);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a16[b][0], b16[b][0][1], acc[1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      tl = tail_mma<2>(a4[b], b4[b][1], tl);
+      tl = tail_mma<3>(a4[b], b4[b][1], tl);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a16[b][1], b16[b][1][0], acc[0], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      tl = tail_mma<4>(a4[b], b4[b][2], tl);
+      tl = tail_mma<5>(a4[b], b4[b][2], tl);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a16[b][1], b16[b][1][1], acc[1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      tl = tail_mma<6>(a4[b], b4[b][3], tl);
+      tl = tail_mma<7>(a4[b], b4[b][3], tl);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // the chunk is in; a barrier with no fence, after which every wave is done
+  // with the other stage, refilled with the next chunk
+  auto body = [&](const float* st, float* other, int ch) {
+    wait_vmcnt<0>();
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+    if (ch + 1 < nch) issue(ch + 1, other);
+    mma(st);
+  };
+  for (int ch = 0; ch < nch; ch += 2) {
+    body(s0, s1, ch);
+    if (ch + 1 < nch) body(s1, s0, ch + 1);
+  }
+
+  auto finish = [&](float x, float b) {
+    x = x + b;
+    if constexpr (AK == 2)
+      x = relu1(x);
+    else if constexpr (AK < 0)
+      x = act_apply(x, p.act);
+    return x;
+  };
+  if constexpr (CVT) {
+    // the outputs go to the stage the last chunk did not use, the ConvT
+    // weights, once every wave is done with it, to the other
+    float* fa = nch & 1 ? s1 : s0;
+    float* fb = nch & 1 ? s0 : s1;
+    float* hh = fa + wave * 32 * CV_HP;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      hh[l16 * CV_HP + 4 * lg + v] = finish(acc[0][v], bterm[v]);
+      hh[(16 + l16) * CV_HP + 4 * lg + v] = finish(acc[1][v], bterm[v]);
+      hh[l32 * CV_HP + 16 + 4 * lh + v] = finish(tl[v], bterm[4 + v]);
+    }
+    __syncthreads();
+    convt_finish<2>(p, cv, hh, fb, w1r, w2r, wave, lane, img, poy, ox0 + l16);
+    return;
+  }
+  if (poy >= p.oh) return;
+  const int64_t yoh = (int64_t)p.oh * p.y_up, yow = (int64_t)p.ow * p.y_up;
+  float* ybase = p.y + ((int64_t)img * p.y_ctotal + p.y_coff) * yoh * yow;
+  const float* rbase = p.res ? p.res + ((int64_t)img * p.m * p.oh + poy) * p.ow : nullptr;
+  float outv[3][4];   // the two tiles of channels 0-15, then channels 16-23
+#pragma unroll
+  for (int g = 0; g < 3; g++) {
+    const int pox = ox0 + (g == 2 ? l32 : 16 * g + l16);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int co = g == 2 ? 16 + 4 * lh + v : 4 * lg + v;
+      float x = finish(g == 2 ? tl[v] : acc[g & 1][v], bterm[(g == 2 ? 4 : 0) + v]);
+      if (rbase && co < p.m && pox < p.ow) x = x + rbase[(int64_t)co * p.oh * p.ow + pox];
+      outv[g][v] = x;
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 3; g++) {
+    const int pox = ox0 + (g == 2 ? l32 : 16 * g + l16);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int co = g == 2 ? 16 + 4 * lh + v : 4 * lg + v;
+      if (co < p.m && pox < p.ow)
+        store_replicated(ybase + (int64_t)co * yoh * yow, yow, poy, pox, (int)p.y_up, outv[g][v]);
+    }
+  }
+}
+
+template <int AK, bool NARROW>
+__global__ __launch_bounds__(256, 3) void conv3x3_tall_kernel(LdsConvGroup g) {
+  __shared__ __attribute__((aligned(16))) float s0[LT_STAGE], s1[LT_STAGE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+  const int t = blockIdx.x;
+  const int i = (t >= g.start[1]) + (t >= g.start[2]) + (t >= g.start[3]);
+  tall_conv_tile<AK, false, NARROW>(g.k[i], g.tiles_x[i], t - g.start[i], s0, s1, wave, lane);
+}
+
+template <int AK>
+__global__ __launch_bounds__(256, 3) void conv3x3_tall_convt_kernel(DirectConvK k, int tiles_x,
+                                                                 ConvtEpi cv) {
+  __shared__ __attribute__((aligned(16))) float s0[LT_STAGE], s1[LT_STAGE];
+  static_assert(4 * 32 * CV_HP <= LT_STAGE && 4 * CV_C * CV_C + 4 * CV_C <= LT_STAGE, "");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+  tall_conv_tile<AK, true, false>(k, tiles_x, blockIdx.x, s0, s1, wave, lane, cv);
 }
 
 // One plain 32-channel conv (no residual, no upsampled store, no activation
@@ -1026,18 +1325,39 @@ static bool lds3x3_pays(const ConvArgs* a, int n) {
   return !narrow || tiles >= LDS_NARROW_TILES;
 }
 
+// Whether the tall kernel takes them (lds3x3_pays already holds): from some two
+// workgroups a CU on (at 428 tiles, the neck of a 960x544 page, it took 45 us
+// against 41).
+#define TALL_MIN_TILES 480
+static bool tall3x3_pays(const ConvArgs* a, int n) {
+  int64_t tiles = 0;
+  for (int i = 0; i < n; i++) {
+    if (a[i].m <= 16 || a[i].m > LT_WC) return false;
+    tiles += (int64_t)ceil_div(a[i].ow, 32) * ceil_div(a[i].oh, 4) * a[i].n;
+  }
+  return tiles >= TALL_MIN_TILES;
+}
+
+template <int AK>
+static void launch_tall(const LdsConvGroup& g, dim3 grid, bool narrow, hipStream_t s) {
+  if (narrow)
+    hipLaunchKernelGGL((conv3x3_tall_kernel<AK, true>), grid, dim3(256), 0, s, g);
+  else
+    hipLaunchKernelGGL((conv3x3_tall_kernel<AK, false>), grid, dim3(256), 0, s, g);
+}
+
 static int launch_lds3x3(const ConvArgs* a, int n, hipStream_t s) {
   LdsConvGroup g{};
   g.n = n;
   int64_t total = 0;
   bool narrow = false;
+  const bool tall = tall3x3_pays(a, n);
   for (int i = 0; i < n; i++) {
     direct_params(a[i], a[i].wk, g.k[i]);
-    g.narrow[i] = !lds3x3_wide(a[i]);
-    narrow = narrow || g.narrow[i];
+    narrow = narrow || !lds3x3_wide(a[i]);
     g.tiles_x[i] = (int)ceil_div(a[i].ow, 32);
     g.start[i] = (int)total;
-    total += (int64_t)g.tiles_x[i] * ceil_div(a[i].oh, 2) * a[i].n;
+    total += (int64_t)g.tiles_x[i] * ceil_div(a[i].oh, tall ? 4 : 2) * a[i].n;
   }
   for (int i = n; i <= DIRECT_GROUP_MAX; i++) g.start[i] = (int)total;
   if (total >= (1ll << 31)) return fail(QPH_EUNSUPPORTED, "conv: grid too large");
@@ -1045,7 +1365,7 @@ static int launch_lds3x3(const ConvArgs* a, int n, hipStream_t s) {
   for (int i = 1; i < n; i++)
     if (a[i].act.kind != kind) kind = -1;
   const dim3 grid((unsigned)total);
-  if (n == 1 && !narrow && a[0].c == 32 && (kind == 0 || kind == 2) && !a[0].res && a[0].y_up == 1 &&
+  if (n == 1 && !narrow && !tall && a[0].c == 32 && (kind == 0 || kind == 2) && !a[0].res && a[0].y_up == 1 &&
       a[0].y_ctotal < (1ll << 31) && a[0].y_coff < (1ll << 31)) {
     const DirectConvK& k = g.k[0];
     if (kind == 0)
@@ -1055,6 +1375,15 @@ static int launch_lds3x3(const ConvArgs* a, int n, hipStream_t s) {
       hipLaunchKernelGGL(conv3x3_lds32_kernel<2>, grid, dim3(256), 0, s, k.x, k.wk, k.bias, k.y,
                          k.h, k.w, k.m, g.tiles_x[0], (int)k.y_ctotal, (int)k.y_coff);
     return launch_check("conv3x3_lds32_kernel");
+  }
+  if (tall) {
+    if (kind == 0)
+      launch_tall<0>(g, grid, narrow, s);
+    else if (kind == 2)
+      launch_tall<2>(g, grid, narrow, s);
+    else
+      launch_tall<-1>(g, grid, narrow, s);
+    return launch_check("conv3x3_tall_kernel");
   }
   if (kind == 0)
     launch_lds_ring<0>(g, grid, narrow, s);
@@ -1082,10 +1411,17 @@ int launch_conv3x3_convt(const ConvArgs& a, const float* w1, const float* w2, fl
   DirectConvK k{};
   direct_params(a, a.wk, k);
   const int tiles_x = (int)ceil_div(a.ow, 32);
-  const int64_t total = (int64_t)tiles_x * ceil_div(a.oh, 2) * a.n;
+  const bool tall = tall3x3_pays(&a, 1);
+  const int64_t total = (int64_t)tiles_x * ceil_div(a.oh, tall ? 4 : 2) * a.n;
   if (total >= (1ll << 31)) return fail(QPH_EUNSUPPORTED, "conv: grid too large");
   const ConvtEpi cv{w1, w2, y};
-  if (a.act.kind == 2)
+  if (tall && a.act.kind == 2)
+    hipLaunchKernelGGL(conv3x3_tall_convt_kernel<2>, dim3((unsigned)total), dim3(256), 0, s, k,
+                       tiles_x, cv);
+  else if (tall)
+    hipLaunchKernelGGL(conv3x3_tall_convt_kernel<0>, dim3((unsigned)total), dim3(256), 0, s, k,
+                       tiles_x, cv);
+  else if (a.act.kind == 2)
     hipLaunchKernelGGL(conv3x3_lds_convt_kernel<2>, dim3((unsigned)total), dim3(256), 0, s, k,
                        tiles_x, cv);
   else

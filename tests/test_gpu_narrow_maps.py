@@ -1,7 +1,8 @@
 """Convs of maps whose rows are not 16-byte aligned or whole: the pointwise
 kernel's one-word slab loads (1 to 512 output channels) and the LDS 3x3
-kernel's one-word halo loads, and a det net with such coarse levels (grouped
-laterals and smoothing convs).  Bit-exact against the oracle."""
+kernel's one-word halo loads, the 3x3 kernel of large maps with 17 to 24
+outputs, and det nets that take all of them (grouped laterals and smoothing
+convs, the head's conv-transpose pair).  Bit-exact against the oracle."""
 import numpy as np
 import pytest
 
@@ -45,7 +46,14 @@ def test_conv3x3_any_width(gpu, oracle, n, c, h, w, m, res):
     _conv(gpu, oracle, n, c, h, w, m, 3, res)
 
 
-@pytest.mark.parametrize("h,w", [(96, 160), (224, 416)])
+@pytest.mark.parametrize("n,c,h,w,m,res", [
+    (1, 8, 481, 97, 24, True), (1, 16, 477, 128, 17, False),   # 484 and 480 tiles
+    (3, 24, 161, 124, 23, False), (1, 40, 479, 100, 20, True), (2, 32, 240, 127, 24, False)])
+def test_conv3x3_tall(gpu, oracle, n, c, h, w, m, res):
+    _conv(gpu, oracle, n, c, h, w, m, 3, res)
+
+
+@pytest.mark.parametrize("h,w", [(96, 160), (224, 416), (960, 992)])
 def test_det_net_odd_coarse_levels(gpu, oracle, h, w):
     from qppocr_amd import nets
     from oracle import nets as onets
