@@ -637,27 +637,25 @@ static void launch_pw_w(int mbw, const GemmArgs& g, int mgroups, dim3 grid, hipS
   switch (mbw) {
     case 1: launch_pw_m<1, WIDE>(g, mgroups, grid, deep, s); break;
     case 2: launch_pw_m<2, WIDE>(g, mgroups, grid, deep, s); break;
-    case 3: launch_pw_m<3, WIDE>(g, mgroups, grid, deep, s); break;
-    case 4: launch_pw_m<4, WIDE>(g, mgroups, grid, deep, s); break;
-    case 5: launch_pw_m<5, WIDE>(g, mgroups, grid, deep, s); break;
-    case 6: launch_pw_m<6, WIDE>(g, mgroups, grid, deep, s); break;
-    case 7: launch_pw_m<7, WIDE>(g, mgroups, grid, deep, s); break;
-    default: launch_pw_m<8, WIDE>(g, mgroups, grid, deep, s); break;
+    default: launch_pw_m<3, WIDE>(g, mgroups, grid, deep, s); break;
   }
 }
 
 static int launch_pw(const GemmArgs& g, hipStream_t s) {
   const int mb = (int)ceil_div(g.m, 16);
   const int64_t pgroups = ceil_div(g.n, 16);
-  // blocks per wave: the most, up to 8, that still leave >= 2048 waves (else
-  // 1) and at most one block in nine past M: more blocks share one X slab,
-  // fewer spread the chains
+  // Row blocks per wave.  A wave holds few loads in flight, so many short waves
+  // beat fewer long ones until the X slabs they re-read cost more: one block,
+  // two from 16384 waves (from 4096 at K >= 128), three at K >= 256.  In us with
+  // one, two and three blocks: 96x147456x32 41.8, 38.3, 39.4 (six: 53.2);
+  // 96x57600x32 17.7, 18.0, 18.1 (six: 27.0); 96x25921x64 15.4, 16.9, 17.4;
+  // 256x10000x256 27.7, 27.8, 33.2; 96x25600x256 36.7, 31.9, 29.3.
+  auto waves = [&](int c) { return pgroups * (int64_t)ceil_div(mb, c) * g.batch; };
   int mbw = 1;
-  for (int c = mb < 8 ? mb : 8; c >= 1; c--)
-    if ((ceil_div(mb, c) * c - mb) * 8 <= mb && pgroups * ceil_div(mb, c) * g.batch >= 2048) {
-      mbw = c;
-      break;
-    }
+  if (g.k >= 256 && mb % 3 == 0 && waves(3) >= 2048)
+    mbw = 3;
+  else if (waves(2) >= 16384 || (g.k >= 128 && waves(2) >= 4096))
+    mbw = 2;
   const int mgroups = (int)ceil_div(mb, mbw);
   if (pgroups * mgroups >= (1ll << 31)) return fail(QPH_EUNSUPPORTED, "gemm: grid too large");
   dim3 grid((unsigned)(pgroups * mgroups), 1, (unsigned)g.batch);

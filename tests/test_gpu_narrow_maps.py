@@ -32,7 +32,9 @@ def _conv(gpu, oracle, n, c, h, w, m, k, res):
 @pytest.mark.parametrize("n,c,h,w,m,res", [
     (1, 16, 1, 1, 1, False), (1, 16, 1, 15, 16, True), (2, 48, 1, 17, 17, False),
     (3, 32, 5, 13, 96, True), (1, 256, 5, 13, 96, False), (1, 64, 33, 33, 129, False),
-    (2, 32, 7, 9, 300, True), (1, 32, 151, 151, 151, False),   # 7 row blocks of 10: two past M
+    (2, 32, 7, 9, 300, True), (1, 32, 151, 151, 151, False),
+    (1, 16, 520, 512, 40, False),     # two row blocks a wave, one past M
+    (2, 128, 101, 163, 96, True), (1, 256, 129, 129, 96, False),   # two, three
     (1, 16, 200, 103, 512, False), (4, 128, 6, 6, 512, True)])
 def test_conv1x1_any_map(gpu, oracle, n, c, h, w, m, res):
     _conv(gpu, oracle, n, c, h, w, m, 1, res)
