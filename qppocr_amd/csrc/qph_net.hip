@@ -889,6 +889,8 @@ static int plan_fpn(qph_net* net) {
     if (!ok) continue;
     const int64_t* s3 = &net->shapes[4 * (size_t)q[2]->out];
     if (s3[2] % 4 || s3[3] % 4) continue;
+    // (the top-down pass counts its elements in 31 bits)
+    if (numel_of(net, q[2]->out) >= (1ll << 31) || (uintptr_t)net->tptr[q[2]->out] % 16) continue;
     // the grouped GEMMs at the full batch take the pointwise group kernel
     for (int k = 0; k < 3 && ok; k++) {
       GemmArgs g{};
