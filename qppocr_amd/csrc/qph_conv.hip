@@ -709,12 +709,12 @@ __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x,
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
       if (NARROW && halo)
-        __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds),
+        __asm__ volatile(QPH_M0 "buffer_load_dword %1, %2, %3 offen lds" ::"s"(lds),
                          "v"(doff[q]), "s"(xr), "s"(soff)
                          : "m0");
       else
         __asm__ volatile(
-            "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
+            QPH_M0 "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
             "v"(doff[q]), "s"(halo ? xr : wr), "s"(soff)
             : "m0");
 #pragma clang diagnostic pop
@@ -1044,12 +1044,12 @@ __device__ __forceinline__ void tall_conv_tile(const DirectConvK& p, int tiles_x
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
       if (NARROW && halo)
-        __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds),
+        __asm__ volatile(QPH_M0 "buffer_load_dword %1, %2, %3 offen lds" ::"s"(lds),
                          "v"(doff[q]), "s"(xr), "s"(soff)
                          : "m0");
       else
         __asm__ volatile(
-            "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
+            QPH_M0 "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
             "v"(doff[q]), "s"(halo ? xr : wr), "s"(soff)
             : "m0");
 #pragma clang diagnostic pop

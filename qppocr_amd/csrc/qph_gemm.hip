@@ -398,20 +398,20 @@ __device__ __forceinline__ void pw_tile(const GemmArgs& g, int mgroups, int blk,
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
     if constexpr (WIDE) {
-      __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lx),
+      __asm__ volatile(QPH_M0 "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lx),
                        "v"(xoff), "s"(xr), "s"(sx)
                        : "m0");
     } else {
 #pragma unroll
       for (int x = 0; x < XL; x++)
-        __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(
+        __asm__ volatile(QPH_M0 "buffer_load_dword %1, %2, %3 offen lds" ::"s"(
                              lx + 256u * x),
                          "v"(xoff), "s"(xr), "s"(sx + x * (xstep >> 2))
                          : "m0");
     }
 #pragma unroll
     for (int w = 0; w < MBW; w++)
-      __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(
+      __asm__ volatile(QPH_M0 "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(
                            lx + 1024u * (1 + w)),
                        "v"(woff[w]), "s"(wr), "s"(sw)
                        : "m0");

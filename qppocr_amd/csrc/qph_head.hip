@@ -306,7 +306,7 @@ head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rs
       const unsigned soff = (unsigned)((b0 + b) * HS_BLOCK + q * 1024);
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
-      __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst),
+      __asm__ volatile(QPH_M0 "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst),
                        "v"(voff), "s"(wr), "s"(soff)
                        : "m0", "memory");
 #pragma clang diagnostic pop

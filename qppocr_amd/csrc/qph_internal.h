@@ -271,6 +271,11 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0xF << 8));
 }
 
+// The head of an inline-asm load to LDS: m0 = operand 0 (the LDS byte address),
+// and the wait state that a scalar write of m0 needs before such a load reads
+// it (the compiler inserts it for its own code, not inside an asm string).
+#define QPH_M0 "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+
 // Reference bias placement (gemm.rs:7-16): rule 0 (panel kernel): seeded
 // when row is in the M%4 tail and the 32-column panel is partial; rule 1
 // (m-rows kernel): seeded for columns j >= n - n%32.

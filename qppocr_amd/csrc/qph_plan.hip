@@ -597,7 +597,7 @@ __global__ __launch_bounds__(64) void plan_conv_dma_kernel(ConvK p) {
           (unsigned)(uintptr_t)(__attribute__((address_space(3))) float4*)(buf + 64 * i));
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
-      __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m),
+      __asm__ volatile(QPH_M0 "buffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m),
                        "v"(off), "s"(isx ? xr : wr)
                        : "m0");
 #pragma clang diagnostic pop
@@ -888,7 +888,7 @@ __device__ __forceinline__ void plan_conv_halo_tile(const ConvK& p, int tiles_x,
           (unsigned)(uintptr_t)(__attribute__((address_space(3))) float4*)(buf + 64 * (L * wave + i)));
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
-      __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m),
+      __asm__ volatile(QPH_M0 "buffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m),
                        "v"(o), "s"(isx ? xr : wr)
                        : "m0");
 #pragma clang diagnostic pop

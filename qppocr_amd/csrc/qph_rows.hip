@@ -1231,7 +1231,7 @@ __global__ __launch_bounds__(512) void qkv_attention_kernel(const float* __restr
           (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)(st + 256 * (5 * wave + u)));
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved; nothing else uses it here
-      __asm__ volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m),
+      __asm__ volatile(QPH_M0 "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m),
                        "v"(off[u]), "s"(isx ? xr : wr), "s"(so)
                        : "m0");
 #pragma clang diagnostic pop
