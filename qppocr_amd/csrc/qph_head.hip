@@ -18,10 +18,11 @@
 // falls from 2.1 to 1.7 GHz (3930 cycles a block of 32 columns, 2.3 us; the bare
 // products 3445 cycles at 1.72 GHz); below some 64 rows the 19 MB of weight.
 //
-// Rows that hold an infinity, a NaN or a magnitude past 2^60 are flagged and
-// recomputed by the pairs kernel in float32, in the order of the unsplit
-// kernels (gemm_wave_kernel, head_pairs_kernel); a weight or bias that holds
-// one keeps the session on those kernels altogether.
+// Rows that hold an infinity, a NaN or a magnitude past 2^60, or whose products
+// with the weight may pass 2^100, are flagged and recomputed by the pairs kernel
+// in float32, in the order of the unsplit kernels (gemm_wave_kernel,
+// head_pairs_kernel); a weight or bias that holds an infinity, a NaN or a
+// magnitude past 2^60 keeps the session on those kernels altogether.
 #include <cmath>
 #include <algorithm>
 #include <vector>
@@ -42,6 +43,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define HS_MAX_LEN 224                 // most column blocks of a slice (their scales sit in LDS)
 #define HS_SMALL 64                    // rows up to which each wave streams its own block
 #define HS_LIMIT 1.152921504606847e18f // 2^60
+#define HS_PRODUCT 1.2676506e30f       // 2^100: the largest |x| |w| a split row may have
 #define HS_L2E 1.44269504f
 
 // 2^(14 - exponent of mx), so that mx times it lies in [2^14, 2^15); the
@@ -56,15 +58,14 @@ __device__ __forceinline__ float pow2_scale(float mx) {
 // and term (h, l), the 64 lanes' eight float16 (lane L: column L % 32, k = 16
 // ks + 8 (L / 32) ..), so a lane's operand is one 16-byte read and a wave's
 // 1024 contiguous bytes.  ci: per column (2^-s log2 e, bias log2 e), past N (0, -3e38):
-// such a column's exponential is 0 beside any other.  w0: column 0 and its
-// bias, times log2 e.  flag[cb]: 1 where the
-// block cannot be split (infinity, NaN, past 2^60).
+// such a column's exponential is 0 beside any other.  top[cb]: the block's
+// largest magnitude, -1 where the block cannot be split (infinity, NaN, past
+// 2^60).
 __global__ __launch_bounds__(256) void head_pack_kernel(const float* __restrict__ w, int n,
                                                         const float* __restrict__ bias,
                                                         _Float16* __restrict__ wp,
                                                         float2* __restrict__ ci,
-                                                        float* __restrict__ w0,
-                                                        int* __restrict__ flag) {
+                                                        float* __restrict__ top) {
   __shared__ float t[HS_K * 33];
   __shared__ float mxs[8 * 32];
   __shared__ float scs[32];
@@ -95,10 +96,9 @@ __global__ __launch_bounds__(256) void head_pack_kernel(const float* __restrict_
     o.x = j < n ? (1.0f / s) * HS_L2E : 0.0f;
     o.y = j < n ? b * HS_L2E : -3.0e38f;
     ci[j] = o;
-    if (j == 0) w0[HS_K] = o.y;
+    mxs[c] = mx;
   }
   __syncthreads();
-  if (cb == 0) w0[tid] = t[tid * 33] * HS_L2E;
   for (int q = tid; q < HS_KS * 64; q += 256) {
     const int ks = q >> 6, lane = q & 63;
     const int col = lane & 31, k0 = 16 * ks + 8 * (lane >> 5);
@@ -113,22 +113,23 @@ __global__ __launch_bounds__(256) void head_pack_kernel(const float* __restrict_
     o[0] = h;
     o[64] = l;
   }
-  if (tid == 0) flag[cb] = bad;
+  if (tid == 0) {
+    for (int q = 1; q < 32; q++) mx = fmaxf(mx, mxs[q]);
+    top[cb] = bad ? -1.0f : mx;
+  }
 }
 
 // The rows of x as split MFMA operands, one workgroup per 32 rows: xs holds per
 // row tile and step ks the h and the l terms of the 64 lanes (lane L: row
 // L % 32, k = 16 ks + 8 (L / 32) ..), so that a wave reads 1 KB at a time; rs
-// holds each row's (2^-s, ref): -1 for a flagged row (whose terms are 0), and
-// the row's logit of column 0 (w0: that column and its bias, times log2 e),
-// which its exponentials are taken against.  Rows past m
-// repeat the last one.  Made once per run in a launch of its own (4.8 us at 1280
-// rows): splitting its own rows cost every workgroup of the product about 10 us
-// (strided reads, some 1300 conversions a lane).
+// holds each row's 2^-s, -1 for a flagged row (whose terms are 0); wmax is the
+// weight's largest magnitude.  Rows past m repeat the last one.  Made once per
+// run in a launch of its own (4.8 us at 1280 rows): splitting its own rows cost
+// every workgroup of the product about 10 us (strided reads, some 1300
+// conversions a lane).
 __global__ __launch_bounds__(256) void head_rows_kernel(const float* __restrict__ x, int m,
-                                                        const float* __restrict__ w0,
-                                                        _Float16* __restrict__ xs,
-                                                        float2* __restrict__ rs) {
+                                                        float wmax, _Float16* __restrict__ xs,
+                                                        float* __restrict__ rs) {
   typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
   const int tid = threadIdx.x, r = tid >> 3, c = tid & 7;
   const float* xr = x + (int64_t)min((int)blockIdx.x * 32 + r, m - 1) * HS_K + 4 * c;
@@ -150,13 +151,10 @@ __global__ __launch_bounds__(256) void head_rows_kernel(const float* __restrict_
     mx = fmaxf(mx, __shfl_xor(mx, off, 64));
     odd |= __shfl_xor(odd, off, 64);
   }
+  odd |= !(mx * wmax <= HS_PRODUCT);
   const float s = pow2_scale(mx);
-  float ref = 0.0f;
 #pragma unroll
   for (int i = 0; i < HS_K / 32; i++) {
-    const f32x4 wq = *(const f32x4*)(w0 + 32 * i + 4 * c);
-#pragma unroll
-    for (int u = 0; u < 4; u++) ref = __builtin_fmaf(raw[i][u], wq[u], ref);
     h16x4 h, l;
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -170,14 +168,7 @@ __global__ __launch_bounds__(256) void head_rows_kernel(const float* __restrict_
     *(h16x4*)o = h;
     *(h16x4*)(o + 512) = l;
   }
-#pragma unroll
-  for (int off = 4; off >= 1; off >>= 1) ref += __shfl_xor(ref, off, 64);
-  if (c == 0) {
-    float2 o;
-    o.x = odd ? -1.0f : 1.0f / s;
-    o.y = odd ? 0.0f : ref + w0[HS_K];
-    rs[blockIdx.x * 32 + r] = o;
-  }
+  if (c == 0) rs[blockIdx.x * 32 + r] = odd ? -1.0f : 1.0f / s;
 }
 
 // A wave's operands of one step of a row tile, from xs.
@@ -188,11 +179,11 @@ __device__ __forceinline__ void load_rows(const _Float16* __restrict__ xs, int t
   al = p[64];
 }
 
-// Running (max, block of the first max, sum of exponentials against the row's
-// ref) of one row's columns lane % 32, 32 + lane % 32, ..., all in powers of
-// two.  ref is the row's logit of column 0, so the row's whole sum is at least 1
-// and overflows only where another logit is 2^127 times as likely (state_store
-// flags such a row); a sum that underflows is nothing beside that 1.
+// Running (max, block of the first max, sum of exponentials against that max)
+// of one row's columns lane % 32, 32 + lane % 32, ..., all in powers of two.  A
+// sum is taken against its own running max, so it lies between 1 and the
+// column count whatever the row's logits are.  (Columns past N alone leave a max
+// of -3e38, whose sum the first real column's exponential, 0, clears.)
 struct RowState {
   float m[16], s[16];
   int b[16];
@@ -209,11 +200,13 @@ __device__ __forceinline__ void state_init(RowState& st) {
 
 // Value v of a block's 32x32 accumulators (lane: column L % 32, rows 8 (v / 4) +
 // 4 (L / 32) + v % 4).
-__device__ __forceinline__ void state_add(RowState& st, int v, float acc, float sr, float ref,
-                                          float2 c, int blk) {
+__device__ __forceinline__ void state_add(RowState& st, int v, float acc, float sr, float2 c,
+                                          int blk) {
   const float t = __builtin_fmaf(acc * sr, c.x, c.y);
-  st.s[v] += __builtin_amdgcn_exp2f(t - ref);
+  // the lesser of the two against the larger: one exponential either way
+  const float e = __builtin_amdgcn_exp2f(-__builtin_fabsf(t - st.m[v]));
   const bool up = t > st.m[v];
+  st.s[v] = __builtin_fmaf(st.s[v], up ? e : 1.0f, up ? 1.0f : e);
   st.b[v] = up ? blk : st.b[v];
   st.m[v] = up ? t : st.m[v];
 }
@@ -221,16 +214,11 @@ __device__ __forceinline__ void state_add(RowState& st, int v, float acc, float 
 // The 32 lanes of each half meet, each step halving the rows a lane still
 // holds; then lane 2 v of a half stores row v's (max, first column of the max,
 // sum, flag).
-__device__ __forceinline__ void state_store(RowState& st, const float2* rw, int m, int row,
+__device__ __forceinline__ void state_store(RowState& st, const float* rw, int m, int row,
                                             int slices, int slice, float* __restrict__ part) {
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
 #pragma unroll
-  for (int v = 0; v < 16; v++) {
-    st.b[v] = st.b[v] * 32 + lr;
-    // (an infinite sum stays infinite or becomes NaN on the way to the store)
-    const float f = __builtin_amdgcn_exp2f(rw[8 * (v >> 2) + 4 * lh + (v & 3)].y - st.m[v]);
-    st.s[v] = st.s[v] > 0.0f ? st.s[v] * f : 0.0f;
-  }
+  for (int v = 0; v < 16; v++) st.b[v] = st.b[v] * 32 + lr;
   auto meet = [&](int v, float mo, float so, int io) {
     const float mm = fmaxf(st.m[v], mo);
     st.s[v] = st.s[v] * __builtin_amdgcn_exp2f(st.m[v] - mm) +
@@ -263,7 +251,7 @@ __device__ __forceinline__ void state_store(RowState& st, const float2* rw, int 
     o[0] = st.m[0];
     o[1] = __int_as_float(st.b[0]);
     o[2] = st.s[0];
-    o[3] = rw[r].x < 0.0f || !(st.s[0] < 3.0e38f) ? 1.0f : 0.0f;
+    o[3] = rw[r] < 0.0f ? 1.0f : 0.0f;   // flagged, in every slice alike
     *(f32x4*)(part + ((int64_t)(row + r) * slices + slice) * 4) = o;
   }
 }
@@ -277,7 +265,7 @@ __device__ __forceinline__ void state_store(RowState& st, const float2* rw, int 
 // wave and eight waves the same LDS reads fed half as many products, and the two
 // waves of a SIMD fell into step with each other: 3.0 us a block.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void
-head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rsc, int m,
+head_split_kernel(const _Float16* __restrict__ xs, const float* __restrict__ rsc, int m,
                   const _Float16* __restrict__ wp, const float2* __restrict__ ci, int nb,
                   int tiles, int slices, int share, int extra, int per_xcd,
                   float* __restrict__ part) {
@@ -291,8 +279,8 @@ head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rs
   const int len = share + (slice < extra ? 1 : 0);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, lr = lane & 31;
-  float2* srl = (float2*)(lds + HS_STAGES * HS_BLOCK);   // (scale, ref) per row
-  float2* cil = srl + HS_ROWS;
+  float* srl = (float*)(lds + HS_STAGES * HS_BLOCK);   // the rows' scales
+  float2* cil = (float2*)(srl + HS_ROWS);
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)wp, 0, nb * HS_BLOCK, 0x00020000);
   // eight 1 KB loads a wave and stage (the asm keeps the compiler from waiting
@@ -339,8 +327,8 @@ head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rs
   }
   issue(0, 0);
   if (len > 1) issue(1, 1);
-  const float2* rw = srl + wave * 64;
-  const float2* rh = rw + 4 * (lane >> 5);
+  const float* rw = srl + wave * 64;
+  const float* rh = rw + 4 * (lane >> 5);
   RowState rs[2];
   state_init(rs[0]);
   state_init(rs[1]);
@@ -359,13 +347,13 @@ head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rs
     if (b + 2 < len) issue(b + 2, st == 0 ? 2 : st - 1);
     const h16x8* bs = (const h16x8*)(lds + st * HS_BLOCK) + lane;
     f32x16 acc[2] = {};
-    // operands, scales and refs one step ahead
+    // operands and scales one step ahead
     h16x8 bh = bs[0], bl = bs[64];
-    float2 rq[2] = {rh[0], rh[32]};
+    float rq[2] = {rh[0], rh[32]};
 #pragma unroll
     for (int ks = 0; ks < HS_KS; ks++) {
       h16x8 nh = bh, nl = bl;
-      float2 nq[2] = {rq[0], rq[1]};
+      float nq[2] = {rq[0], rq[1]};
       if (ks + 1 < HS_KS) {
         const int r = 8 * ((ks + 1) >> 2) + ((ks + 1) & 3);
         nh = bs[(ks + 1) * 128];
@@ -387,11 +375,11 @@ head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rs
         acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t][ks], bh, acc[t], 0, 0, 0);
 #pragma unroll
       for (int t = 0; t < 2; t++)
-        state_add(rs[t], ks, prev[t][ks], rq[t].x, rq[t].y, pc, b0 + b - 1);
+        state_add(rs[t], ks, prev[t][ks], rq[t], pc, b0 + b - 1);
 #pragma unroll
       for (int q = 0; q < 6; q++) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
       bh = nh;
@@ -408,10 +396,8 @@ head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rs
 #pragma unroll
   for (int t = 0; t < 2; t++) {
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const float2 q = rh[32 * t + 8 * (v >> 2) + (v & 3)];
-      state_add(rs[t], v, prev[t][v], q.x, q.y, pc, b0 + len - 1);
-    }
+    for (int v = 0; v < 16; v++)
+      state_add(rs[t], v, prev[t][v], rh[32 * t + 8 * (v >> 2) + (v & 3)], pc, b0 + len - 1);
     state_store(rs[t], rw + 32 * t, m, row + 32 * t, slices, slice, part);
   }
 }
@@ -420,12 +406,12 @@ head_split_kernel(const _Float16* __restrict__ xs, const float2* __restrict__ rs
 // straight into registers, all 32 loads of a lane in flight at once (24 rows:
 // 7.5 us, for 19 MB of weight; the row tile form would keep one wave in eight).
 __global__ __launch_bounds__(64) void head_split_small_kernel(const _Float16* __restrict__ xs,
-                                                              const float2* __restrict__ rsc, int m,
+                                                              const float* __restrict__ rsc, int m,
                                                               const _Float16* __restrict__ wp,
                                                               const float2* __restrict__ ci,
                                                               int nb, int tiles, int per_xcd,
                                                               float* __restrict__ part) {
-  __shared__ float2 srl[32];
+  __shared__ float srl[32];
   const int u = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
   if (u >= tiles * nb) return;
   const int cb = u / tiles, row = (u - cb * tiles) * 32;
@@ -453,10 +439,8 @@ __global__ __launch_bounds__(64) void head_split_small_kernel(const _Float16* __
   RowState rs;
   state_init(rs);
 #pragma unroll
-  for (int v = 0; v < 16; v++) {
-    const float2 q = srl[8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)];
-    state_add(rs, v, acc[v], q.x, q.y, c, cb);
-  }
+  for (int v = 0; v < 16; v++)
+    state_add(rs, v, acc[v], srl[8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)], c, cb);
   state_store(rs, srl, m, row, nb, cb, part);
 }
 
@@ -580,7 +564,7 @@ static int64_t part_floats(int64_t m, int64_t n) {
 }
 
 int64_t head_split_scratch_floats(int64_t m, int64_t n) {
-  return part_floats(m, n) + ceil_div(m, 32) * 32 * (HS_K + 2);
+  return part_floats(m, n) + ceil_div(m, 32) * 32 * (HS_K + 1);
 }
 
 // Packs w[256][n] (rows n apart); *out stays NULL for a weight or bias that
@@ -589,19 +573,18 @@ int head_split_pack(const float* w, int64_t n, const float* bias, HeadSplit* out
   const int nb = (int)ceil_div(n, 32);
   char* d = nullptr;
   const size_t wb = (size_t)nb * HS_BLOCK, cb = (size_t)nb * 32 * sizeof(float2);
-  const size_t w0 = (HS_K + 4) * sizeof(float);
-  QPH_TRY_HIP(hipMalloc((void**)&d, wb + cb + w0 + (size_t)nb * 4));
-  int* flag = (int*)(d + wb + cb + w0);
+  QPH_TRY_HIP(hipMalloc((void**)&d, wb + cb + (size_t)nb * 4));
+  float* top = (float*)(d + wb + cb);
   hipLaunchKernelGGL(head_pack_kernel, dim3((unsigned)nb), dim3(256), 0, s, w, (int)n, bias,
-                     (_Float16*)d, (float2*)(d + wb), (float*)(d + wb + cb), flag);
+                     (_Float16*)d, (float2*)(d + wb), top);
   int rc = launch_check("head_pack_kernel");
-  std::vector<int> f((size_t)nb, 0);
+  std::vector<float> f((size_t)nb, 0.0f);
   if (rc == QPH_OK)
-    rc = hip_check(hipMemcpyAsync(f.data(), flag, (size_t)nb * 4, hipMemcpyDeviceToHost, s),
-                   "hipMemcpyAsync(head flags)");
+    rc = hip_check(hipMemcpyAsync(f.data(), top, (size_t)nb * 4, hipMemcpyDeviceToHost, s),
+                   "hipMemcpyAsync(head maxima)");
   if (rc == QPH_OK) rc = hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
   bool odd = false;
-  for (int v : f) odd = odd || v != 0;
+  for (float v : f) odd = odd || v < 0.0f, out->wmax = std::max(out->wmax, v);
   if (rc != QPH_OK || odd) {
     (void)hipFree(d);
     return rc;
@@ -620,10 +603,10 @@ int launch_head_split(const float* x, int64_t m, const HeadSplit& hs, const floa
   const float2* ci = (const float2*)hs.ci;
   // scratch: the split rows, their scales, the partials
   _Float16* xs = (_Float16*)scratch;
-  float2* rs = (float2*)(scratch + (int64_t)rt * 32 * HS_K);
-  float* part = (float*)(rs + (int64_t)rt * 32);
-  hipLaunchKernelGGL(head_rows_kernel, dim3((unsigned)rt), dim3(256), 0, s, x, (int)m,
-                     (const float*)(ci + (int64_t)nb * 32), xs, rs);
+  float* rs = scratch + (int64_t)rt * 32 * HS_K;
+  float* part = rs + (int64_t)rt * 32;
+  hipLaunchKernelGGL(head_rows_kernel, dim3((unsigned)rt), dim3(256), 0, s, x, (int)m, hs.wmax, xs,
+                     rs);
   QPH_TRY(launch_check("head_rows_kernel"));
   int slices = nb;
   if (m <= HS_SMALL) {
@@ -636,7 +619,7 @@ int launch_head_split(const float* x, int64_t m, const HeadSplit& hs, const floa
     slices = split_slices(tiles, nb);
     const int len = (nb + slices - 1) / slices;
     const int per = (int)ceil_div((int64_t)tiles * slices, 8);
-    const size_t shm = HS_STAGES * HS_BLOCK + (HS_ROWS + (size_t)len * 32) * sizeof(float2);
+    const size_t shm = HS_STAGES * HS_BLOCK + HS_ROWS * sizeof(float) + (size_t)len * 32 * sizeof(float2);
     QPH_TRY(allow_full_lds((const void*)head_split_kernel));
     hipLaunchKernelGGL(head_split_kernel, dim3((unsigned)per * 8), dim3(256), shm, s, xs, rs,
                        (int)m, wp, ci, nb, tiles, slices, nb / slices, nb % slices, per, part);

@@ -221,6 +221,7 @@ int launch_head_argmax(const float* x, int64_t m, int64_t k, const float* w, int
 struct HeadSplit {
   char* wp = nullptr;         // owned by the caller (hipFree)
   const float* ci = nullptr;  // inside wp's allocation
+  float wmax = 0.0f;          // the weight's largest magnitude
 };
 bool head_split_eligible(int64_t k, int64_t n);
 int64_t head_split_scratch_floats(int64_t m, int64_t n);   // for every row count up to m

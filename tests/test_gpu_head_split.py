@@ -124,3 +124,47 @@ def test_head_split_refuses_weights_it_cannot_hold(gpu, where):
     t = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
     old = ops.linear_softmax_argmax(t(x), t(w), t(b)).cpu().numpy()
     assert (pairs.view(np.uint32) == old.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("rows", [24, 300])
+def test_head_split_distant_winner(gpu, rows):
+    """A winner far above every other class, in the first blocks and in the
+    last: gaps around the range of a float32 exponential and past it."""
+    n, cols, gaps = 18709, [10, 40, 5000, 18708], [87.5, 88.5, 95.0, 126.0, 200.0, 3000.0]
+    rng, w, b = _weights(n, rows)
+    w *= 0.1
+    w[:4] = w[:, cols] = 0.0
+    w[range(4), cols] = 1.0             # row q of the weight moves class cols[q] alone
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    x[:, :4] = 0.0
+    for i in range(rows):
+        x[i, i % 4] = gaps[i // 4 % len(gaps)] * (-1 if i >= 4 * len(gaps) and i % 3 == 0 else 1)
+    print(f"head split, distant winners, {rows} rows", flush=True)
+    sess = _session(rows, w, b)
+    pairs = sess.run(x.reshape(rows, 1, 1, K))[0].reshape(rows, 2)
+    sess.close()
+    p, idx, gap = _ref(x, w, b)
+    ids = np.ascontiguousarray(pairs[:, 1]).view(np.uint32)
+    assert (ids == idx)[gap > 1e-4].all()
+    # logits of at most 5 beside the winner's, whose own rounding cancels: 1e-5
+    # is some 40 roundings of such a logit
+    assert (np.abs(pairs[:, 0] - p) <= 1e-5 * p).all()
+
+
+@pytest.mark.parametrize("rows", [24, 300])
+def test_head_split_logits_past_float32(gpu, rows):
+    """Operands within their limit whose products are not: column 0 overflows
+    a float32 sum for some rows, and is far above or below for the others."""
+    rng, w, b = _weights(1001, rows)
+    w[:, 0] = 1e18
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    x[3], x[5] = 1.1e18, -1.1e18
+    x[rows - 1] = 1e12
+    print(f"head split, column 0 of 1e18, {rows} rows", flush=True)
+    sess = _session(rows, w, b)
+    pairs = sess.run(x.reshape(rows, 1, 1, K))[0].reshape(rows, 2)
+    sess.close()
+    p, idx, gap = _ref(x, w, b)
+    ids = np.ascontiguousarray(pairs[:, 1]).view(np.uint32)
+    assert (ids == idx)[gap > 1e-4].all()
+    assert (np.abs(pairs[:, 0] - p) <= 1e-5 * p).all()
