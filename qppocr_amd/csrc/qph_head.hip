@@ -19,10 +19,10 @@
 // products 3445 cycles at 1.72 GHz); below some 64 rows the 19 MB of weight.
 //
 // Rows that hold an infinity, a NaN or a magnitude past 2^60, or whose products
-// with the weight may pass 2^100, are flagged and recomputed by the pairs kernel
-// in float32, in the order of the unsplit kernels (gemm_wave_kernel,
-// head_pairs_kernel); a weight or bias that holds an infinity, a NaN or a
-// magnitude past 2^60 keeps the session on those kernels altogether.
+// with the weight may pass 2^100, are flagged and computed in float32
+// (flagged_tile); a weight or bias that holds an infinity, a NaN or a magnitude
+// past 2^60 keeps the session on the unsplit kernels (gemm_wave_kernel,
+// head_pairs_kernel) altogether.
 #include <cmath>
 #include <algorithm>
 #include <vector>
@@ -199,12 +199,18 @@ __device__ __forceinline__ void state_init(RowState& st) {
 }
 
 // Value v of a block's 32x32 accumulators (lane: column L % 32, rows 8 (v / 4) +
-// 4 (L / 32) + v % 4).
+// 4 (L / 32) + v % 4).  F32: of a flagged tile, in natural units (c.y the bias).
+template <bool F32>
+__device__ __forceinline__ float exp_less(float d) {
+  return __builtin_amdgcn_exp2f(F32 ? d * HS_L2E : d);
+}
+
+template <bool F32>
 __device__ __forceinline__ void state_add(RowState& st, int v, float acc, float sr, float2 c,
                                           int blk) {
-  const float t = __builtin_fmaf(acc * sr, c.x, c.y);
+  const float t = F32 ? acc + c.y : __builtin_fmaf(acc * sr, c.x, c.y);
   // the lesser of the two against the larger: one exponential either way
-  const float e = __builtin_amdgcn_exp2f(-__builtin_fabsf(t - st.m[v]));
+  const float e = exp_less<F32>(-__builtin_fabsf(t - st.m[v]));
   const bool up = t > st.m[v];
   st.s[v] = __builtin_fmaf(st.s[v], up ? e : 1.0f, up ? 1.0f : e);
   st.b[v] = up ? blk : st.b[v];
@@ -213,7 +219,8 @@ __device__ __forceinline__ void state_add(RowState& st, int v, float acc, float 
 
 // The 32 lanes of each half meet, each step halving the rows a lane still
 // holds; then lane 2 v of a half stores row v's (max, first column of the max,
-// sum, flag).
+// sum, flag) if the row is flagged (F32) or is not.
+template <bool F32>
 __device__ __forceinline__ void state_store(RowState& st, const float* rw, int m, int row,
                                             int slices, int slice, float* __restrict__ part) {
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
@@ -221,8 +228,7 @@ __device__ __forceinline__ void state_store(RowState& st, const float* rw, int m
   for (int v = 0; v < 16; v++) st.b[v] = st.b[v] * 32 + lr;
   auto meet = [&](int v, float mo, float so, int io) {
     const float mm = fmaxf(st.m[v], mo);
-    st.s[v] = st.s[v] * __builtin_amdgcn_exp2f(st.m[v] - mm) +
-              so * __builtin_amdgcn_exp2f(mo - mm);
+    st.s[v] = st.s[v] * exp_less<F32>(st.m[v] - mm) + so * exp_less<F32>(mo - mm);
     const int first = min(io, st.b[v]);
     st.b[v] = mo > st.m[v] ? io : mo == st.m[v] ? first : st.b[v];
     st.m[v] = mm;
@@ -246,14 +252,56 @@ __device__ __forceinline__ void state_store(RowState& st, const float* rw, int m
   meet(0, __shfl_xor(st.m[0], 1, 64), __shfl_xor(st.s[0], 1, 64), __shfl_xor(st.b[0], 1, 64));
   const int v = lr >> 1;
   const int r = 8 * (v >> 2) + 4 * lh + (v & 3);
-  if (!(lr & 1) && row + r < m) {
+  if (!(lr & 1) && row + r < m && (rw[r] < 0.0f) == F32) {
     f32x4 o;
     o[0] = st.m[0];
     o[1] = __int_as_float(st.b[0]);
     o[2] = st.s[0];
-    o[3] = rw[r] < 0.0f ? 1.0f : 0.0f;   // flagged, in every slice alike
+    o[3] = F32 ? 1.0f : 0.0f;   // (in every slice alike)
     *(f32x4*)(part + ((int64_t)(row + r) * slices + slice) * 4) = o;
   }
+}
+
+// The partials of a tile's flagged rows over column blocks b0 .. b0 + len - 1, in
+// float32: the whole tile's logits on v_mfma_f32_32x32x2f32, whose two k terms are
+// added in order (the fma chain of the unsplit kernels), an infinity or a NaN
+// staying in its own row.  Every slice does its share: one such row among 1280
+// costs a call 70 us and 1280 of them 170 (as much as the unsplit kernels take for
+// the whole head, and half as much again); a wave a row in the pairs kernel took
+// 7.6 ms for the first.
+__device__ __forceinline__ void flagged_tile(const float* __restrict__ x, int m,
+                                             const float* __restrict__ w, int n,
+                                             const float* __restrict__ bias, int row, int b0,
+                                             int len, const float* rw, int slices, int slice,
+                                             float* __restrict__ part) {
+  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+  // operands: lane (row or column L % 32, half L / 32), k = 2 s + half of step s
+  const float* xr = x + (int64_t)min(row + lr, m - 1) * HS_K + lh;
+  float a[HS_K / 2];
+#pragma unroll
+  for (int s = 0; s < HS_K / 2; s++) a[s] = xr[2 * s];
+  RowState st;
+  state_init(st);
+#pragma unroll 1
+  for (int b = b0; b < b0 + len; b++) {
+    const int j = b * 32 + lr, jc = min(j, n - 1);
+    const float* wc = w + (int64_t)lh * n + jc;
+    // the block's loads all in flight (left alone, the scheduler puts most of
+    // them one by one between the products)
+    float q[HS_K / 2];
+#pragma unroll
+    for (int s = 0; s < HS_K / 2; s++) q[s] = wc[(int64_t)(2 * s) * n];
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16 acc = {};
+#pragma unroll
+    for (int s = 0; s < HS_K / 2; s++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], q[s], acc, 0, 0, 0);
+    const float2 c = {0.0f, bias ? bias[jc] : -0.0f};
+#pragma unroll
+    for (int v = 0; v < 16; v++)
+      state_add<true>(st, v, j < n ? acc[v] : -3.0e38f, 0.0f, j < n ? c : float2{0.0f, 0.0f}, b);
+  }
+  state_store<true>(st, rw, m, row, slices, slice, part);
 }
 
 // Workgroup (row tile of 256, slice of the column blocks): each of the four
@@ -268,7 +316,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 head_split_kernel(const _Float16* __restrict__ xs, const float* __restrict__ rsc, int m,
                   const _Float16* __restrict__ wp, const float2* __restrict__ ci, int nb,
                   int tiles, int slices, int share, int extra, int per_xcd,
-                  float* __restrict__ part) {
+                  float* __restrict__ part, const float* __restrict__ x,
+                  const float* __restrict__ w, int n, const float* __restrict__ bias) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   // slice-major over the XCDs: the row tiles of one slice share an XCD's L2;
   // a slice is share blocks, the first `extra` ones one more
@@ -375,7 +424,7 @@ head_split_kernel(const _Float16* __restrict__ xs, const float* __restrict__ rsc
         acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t][ks], bh, acc[t], 0, 0, 0);
 #pragma unroll
       for (int t = 0; t < 2; t++)
-        state_add(rs[t], ks, prev[t][ks], rq[t], pc, b0 + b - 1);
+        state_add<false>(rs[t], ks, prev[t][ks], rq[t], pc, b0 + b - 1);
 #pragma unroll
       for (int q = 0; q < 6; q++) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -397,9 +446,15 @@ head_split_kernel(const _Float16* __restrict__ xs, const float* __restrict__ rsc
   for (int t = 0; t < 2; t++) {
 #pragma unroll
     for (int v = 0; v < 16; v++)
-      state_add(rs[t], v, prev[t][v], rh[32 * t + 8 * (v >> 2) + (v & 3)], pc, b0 + len - 1);
-    state_store(rs[t], rw + 32 * t, m, row + 32 * t, slices, slice, part);
+      state_add<false>(rs[t], v, prev[t][v], rh[32 * t + 8 * (v >> 2) + (v & 3)], pc,
+                       b0 + len - 1);
+    state_store<false>(rs[t], rw + 32 * t, m, row + 32 * t, slices, slice, part);
   }
+  const uint64_t odd = __ballot(rw[lane] < 0.0f);
+#pragma unroll 1
+  for (int t = 0; t < 2 && row + 32 * t < m; t++)
+    if ((unsigned)(odd >> (32 * t)) != 0)
+      flagged_tile(x, m, w, n, bias, row + 32 * t, b0, len, rw + 32 * t, slices, slice, part);
 }
 
 // Up to HS_SMALL rows: a wave per (32 rows, column block), the block's operands
@@ -410,7 +465,10 @@ __global__ __launch_bounds__(64) void head_split_small_kernel(const _Float16* __
                                                               const _Float16* __restrict__ wp,
                                                               const float2* __restrict__ ci,
                                                               int nb, int tiles, int per_xcd,
-                                                              float* __restrict__ part) {
+                                                              float* __restrict__ part,
+                                                              const float* __restrict__ x,
+                                                              const float* __restrict__ w, int n,
+                                                              const float* __restrict__ bias) {
   __shared__ float srl[32];
   const int u = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
   if (u >= tiles * nb) return;
@@ -440,97 +498,50 @@ __global__ __launch_bounds__(64) void head_split_small_kernel(const _Float16* __
   state_init(rs);
 #pragma unroll
   for (int v = 0; v < 16; v++)
-    state_add(rs, v, acc[v], srl[8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)], c, cb);
-  state_store(rs, srl, m, row, nb, cb, part);
+    state_add<false>(rs, v, acc[v], srl[8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)], c, cb);
+  state_store<false>(rs, srl, m, row, nb, cb, part);
+  if (__ballot(srl[lane & 31] < 0.0f) != 0)
+    flagged_tile(x, m, w, n, bias, row, cb, 1, srl, nb, cb, part);
 }
 
-// (max, first index, sum) of columns 64 t .. + 63 of one row in float32, the
-// terms, order and comparisons of gemm_wave_kernel's argmax epilogue.
-__device__ __noinline__ f32x4 row_block_f32(const float* __restrict__ xr,
-                                            const float* __restrict__ w, int n,
-                                            const float* __restrict__ bias, int t) {
-  float mh[2], sh[2];
-  int ih[2];
-  for (int half = 0; half < 2; half++) {
-    const int jb = 64 * t + 32 * half;
-    float v[32];
-#pragma unroll
-    for (int q = 0; q < 32; q++) v[q] = 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < HS_K; k++) {
-      const float a = xr[k];
-#pragma unroll
-      for (int q = 0; q < 32; q++)
-        if (jb + q < n) v[q] = __builtin_fmaf(a, w[(int64_t)k * n + jb + q], v[q]);
-    }
-    float m = -__builtin_inff(), s = 0.0f;
-    int idx = 0x7fffffff;
-#pragma unroll
-    for (int q = 0; q < 32; q++)
-      if (jb + q < n) {
-        v[q] = v[q] + (bias ? bias[jb + q] : -0.0f);
-        if (v[q] > m) {
-          m = v[q];
-          idx = jb + q;
-        }
-      }
-#pragma unroll
-    for (int q = 0; q < 32; q++)
-      if (jb + q < n) s += __builtin_amdgcn_exp2f((v[q] - m) * HS_L2E);
-    mh[half] = m;
-    sh[half] = s;
-    ih[half] = idx;
-  }
-  const float mm = fmaxf(mh[0], mh[1]);
-  f32x4 o;
-  o[0] = mm;
-  o[1] = __int_as_float(mh[1] > mh[0] ? ih[1] : ih[0]);
-  o[2] = sh[0] * __builtin_amdgcn_exp2f((mh[0] - mm) * HS_L2E) +
-         (sh[1] > 0.0f ? sh[1] * __builtin_amdgcn_exp2f((mh[1] - mm) * HS_L2E) : 0.0f);
-  o[3] = 0.0f;
-  return o;
-}
-
-// Per row: the slices' partials to the (value, index) pair, one wave a row.
-// A flagged row's partials are made here instead, one 64-column block a lane
-// and round.
-__global__ __launch_bounds__(256, 4) void head_split_pairs_kernel(
-    const float* __restrict__ part, int64_t rows, int slices, const float* __restrict__ x,
-    const float* __restrict__ w, int n, const float* __restrict__ bias,
-    float* __restrict__ pairs) {
+// Per row: the slices' partials to the (value, index) pair, one wave a row.  A
+// flagged row's are in natural units, and its logits may have no maximum (nothing
+// but -infinity and NaN: the id is 0x7fffffff) or an infinite one: its value is
+// then 1 / 0, as the unsplit kernels give it.
+__global__ __launch_bounds__(256) void head_split_pairs_kernel(const float* __restrict__ part,
+                                                               int64_t rows, int slices,
+                                                               float* __restrict__ pairs) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const f32x4* pr = (const f32x4*)part + row * slices;
-  const bool odd = pr[0][3] != 0.0f;
-  const int nt = odd ? (n + 63) / 64 : slices;
-  const float l2e = odd ? HS_L2E : 1.0f;
-  float m = -__builtin_inff(), sum = 0.0f;
+  float m = -3.0e38f, sum = 0.0f, l2e = 1.0f;
   int idx = 0x7fffffff;
-  for (int t = lane; t < nt; t += 64) {
-    const f32x4 q = odd ? row_block_f32(x + row * HS_K, w, n, bias, t) : pr[t];
+  for (int t = lane; t < slices; t += 64) {
+    const f32x4 q = pr[t];
+    l2e = q[3] != 0.0f ? HS_L2E : 1.0f;
     if (q[0] > m) {
-      sum = (sum > 0.0f ? sum * __builtin_amdgcn_exp2f((m - q[0]) * l2e) : 0.0f) + q[2];
+      sum = sum * __builtin_amdgcn_exp2f((m - q[0]) * l2e) + q[2];
       m = q[0];
       idx = __float_as_int(q[1]);
     } else {
       sum += q[2] * __builtin_amdgcn_exp2f((q[0] - m) * l2e);
     }
   }
+  l2e = __shfl(l2e, 0, 64);   // (a lane past the slices has not seen the flag)
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     const float mo = __shfl_xor(m, off, 64);
     const int io = __shfl_xor(idx, off, 64);
     const float so = __shfl_xor(sum, off, 64);
     const float mm = fmaxf(m, mo);
-    // a lane without partials has sum 0 and max -inf: its term is 0
-    sum = (sum > 0.0f ? sum * __builtin_amdgcn_exp2f((m - mm) * l2e) : 0.0f) +
-          (so > 0.0f ? so * __builtin_amdgcn_exp2f((mo - mm) * l2e) : 0.0f);
+    sum = sum * __builtin_amdgcn_exp2f((m - mm) * l2e) + so * __builtin_amdgcn_exp2f((mo - mm) * l2e);
     if (mo > m || (mo == m && io < idx)) idx = io;
     m = mm;
   }
   if (lane == 0) {
-    pairs[2 * row] = 1.0f / sum;   // the max's exponential is exp2(0) = 1
+    // the max's exponential is exp2(0) = 1
+    pairs[2 * row] = 1.0f / (m > -3.0e38f && m - m == 0.0f ? sum : 0.0f);
     pairs[2 * row + 1] = __int_as_float(idx);
   }
 }
@@ -612,7 +623,7 @@ int launch_head_split(const float* x, int64_t m, const HeadSplit& hs, const floa
   if (m <= HS_SMALL) {
     const int per = (int)ceil_div((int64_t)rt * nb, 8);
     hipLaunchKernelGGL(head_split_small_kernel, dim3((unsigned)per * 8), dim3(64), 0, s, xs, rs,
-                       (int)m, wp, ci, nb, rt, per, part);
+                       (int)m, wp, ci, nb, rt, per, part, x, w, (int)n, bias);
     QPH_TRY(launch_check("head_split_small_kernel"));
   } else {
     const int tiles = (int)ceil_div(m, HS_ROWS);
@@ -622,11 +633,12 @@ int launch_head_split(const float* x, int64_t m, const HeadSplit& hs, const floa
     const size_t shm = HS_STAGES * HS_BLOCK + HS_ROWS * sizeof(float) + (size_t)len * 32 * sizeof(float2);
     QPH_TRY(allow_full_lds((const void*)head_split_kernel));
     hipLaunchKernelGGL(head_split_kernel, dim3((unsigned)per * 8), dim3(256), shm, s, xs, rs,
-                       (int)m, wp, ci, nb, tiles, slices, nb / slices, nb % slices, per, part);
+                       (int)m, wp, ci, nb, tiles, slices, nb / slices, nb % slices, per, part, x, w,
+                       (int)n, bias);
     QPH_TRY(launch_check("head_split_kernel"));
   }
   hipLaunchKernelGGL(head_split_pairs_kernel, dim3(ceil_div(m, 4)), dim3(256), 0, s, part, m,
-                     slices, x, w, (int)n, bias, pairs);
+                     slices, pairs);
   return launch_check("head_split_pairs_kernel");
 }
 
