@@ -5,11 +5,24 @@
 // s a power of two per row of x and per column of w that puts the row's /
 // column's largest magnitude in [2^14, 2^15): h the nearest float16, l the
 // nearest float16 to the exact remainder.  |e| is at most one float32 ulp of v
-// for the elements within 2^-17 of the largest, and 2^-40 of the largest for
-// the smaller ones.  A product keeps h.h, h.l and l.h; each is exact in
-// float32, and v_mfma_f32_32x32x16_f16 adds them into a float32 accumulator:
-// 48 accumulator roundings per logit where the float32 chain has 256.  Against
-// float64 the pair values of the rec net are 2.5e-6 off, the chain's 3.6e-6.
+// (and 0 for three values in four) for the elements within 2^-15 of the largest,
+// and 2^-39 of the largest for the smaller ones.  A product keeps h.h, h.l and l.h;
+// each is exact in float32, and v_mfma_f32_32x32x16_f16 adds them into a float32
+// accumulator: 48 accumulator roundings per logit where the float32 chain has
+// 256.  l.l, left out, is at most 2^-22 of a product (2^-24.6 in the mean square).
+//
+// So a logit of many terms is closer to float64 than the chain's, one of few
+// terms is not, nor one whose terms are all far below the row's largest element
+// (against a weight of 0).  Mean square error of the logits, split / chain, K =
+// 256 terms of normal values: 4.1e-7 / 8.1e-7; operands spread over 2^20: half the
+// chain's as well; 128 nonzero terms 1.0 / 1.3 of a value, 64: 2.1 / 2.05e-7, 16:
+// 8.8 / 5.2e-8, 1: 14.8 / 4.9e-9; a channel of weight 0 at 2^16 times the others
+// 4.3 / 8.1e-7, at 2^20 2.2e-6 / 8.1e-7.  Rows of fewer than HS_TERMS terms, or with
+// a product past HS_PRODUCT (whose small elements could be off by 2^-18 of a logit's
+// unit, in the worst case), are therefore computed in float32 (flagged_tile), and a
+// weight with a column of so few terms keeps the session on the unsplit kernels.
+// The pair values of the rec net are 2.5e-6 off (mean square, relative), the
+// chain's 3.6e-6.
 //
 // What it measured (N = 18709; split rows + product + pairs, traced, against
 // gemm_wave_kernel + head_pairs_kernel): 1280 rows 47.6 us against 128, 6800 rows
@@ -18,11 +31,9 @@
 // falls from 2.1 to 1.7 GHz (3930 cycles a block of 32 columns, 2.3 us; the bare
 // products 3445 cycles at 1.72 GHz); below some 64 rows the 19 MB of weight.
 //
-// Rows that hold an infinity, a NaN or a magnitude past 2^60, or whose products
-// with the weight may pass 2^100, are flagged and computed in float32
-// (flagged_tile); a weight or bias that holds an infinity, a NaN or a magnitude
-// past 2^60 keeps the session on the unsplit kernels (gemm_wave_kernel,
-// head_pairs_kernel) altogether.
+// Rows that hold an infinity, a NaN or a magnitude past 2^60 are flagged and
+// computed in float32 too; a weight or bias that holds one keeps the session on
+// the unsplit kernels (gemm_wave_kernel, head_pairs_kernel) altogether.
 #include <cmath>
 #include <algorithm>
 #include <vector>
@@ -43,7 +54,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define HS_MAX_LEN 224                 // most column blocks of a slice (their scales sit in LDS)
 #define HS_SMALL 64                    // rows up to which each wave streams its own block
 #define HS_LIMIT 1.152921504606847e18f // 2^60
-#define HS_PRODUCT 1.2676506e30f       // 2^100: the largest |x| |w| a split row may have
+#define HS_PRODUCT 4096.0f             // the largest |x| |w| a split row may have
+#define HS_TERMS 96                    // and the fewest terms of a split row or column:
+#define HS_TERM 9.5367431640625e-7f    // elements past 2^-20 of its largest (or none at all)
 #define HS_L2E 1.44269504f
 
 // 2^(14 - exponent of mx), so that mx times it lies in [2^14, 2^15); the
@@ -60,7 +73,7 @@ __device__ __forceinline__ float pow2_scale(float mx) {
 // 1024 contiguous bytes.  ci: per column (2^-s log2 e, bias log2 e), past N (0, -3e38):
 // such a column's exponential is 0 beside any other.  top[cb]: the block's
 // largest magnitude, -1 where the block cannot be split (infinity, NaN, past
-// 2^60).
+// 2^60, a column of few terms).
 __global__ __launch_bounds__(256) void head_pack_kernel(const float* __restrict__ w, int n,
                                                         const float* __restrict__ bias,
                                                         _Float16* __restrict__ wp,
@@ -88,6 +101,9 @@ __global__ __launch_bounds__(256) void head_pack_kernel(const float* __restrict_
   if (odd) bad = 1;
   if (tid < 32) {
     for (int q = 1; q < 8; q++) mx = fmaxf(mx, mxs[q * 32 + c]);
+    int terms = 0;
+    for (int k = 0; k < HS_K; k++) terms += __builtin_fabsf(t[k * 33 + c]) > mx * HS_TERM;
+    if (terms > 0 && terms < HS_TERMS) bad = 1;
     const float s = pow2_scale(mx);
     scs[c] = s;
     const float b = j < n && bias ? bias[j] : 0.0f;
@@ -151,7 +167,14 @@ __global__ __launch_bounds__(256) void head_rows_kernel(const float* __restrict_
     mx = fmaxf(mx, __shfl_xor(mx, off, 64));
     odd |= __shfl_xor(odd, off, 64);
   }
-  odd |= !(mx * wmax <= HS_PRODUCT);
+  int terms = 0;
+#pragma unroll
+  for (int i = 0; i < HS_K / 32; i++)
+#pragma unroll
+    for (int u = 0; u < 4; u++) terms += __builtin_fabsf(raw[i][u]) > mx * HS_TERM;
+#pragma unroll
+  for (int off = 4; off >= 1; off >>= 1) terms += __shfl_xor(terms, off, 64);
+  odd |= !(mx * wmax <= HS_PRODUCT) || (terms > 0 && terms < HS_TERMS);
   const float s = pow2_scale(mx);
 #pragma unroll
   for (int i = 0; i < HS_K / 32; i++) {

@@ -216,8 +216,9 @@ int launch_head_argmax(const float* x, int64_t m, int64_t k, const float* w, int
                        int64_t n, const float* bias, float* part, float* pairs, hipStream_t s);
 
 // The same over a weight packed once as float16 pairs (qph_head.hip): K = 256,
-// closer to float64 than the float32 chain.  head_split_pack leaves wp NULL
-// for a weight or bias that cannot be split (infinities, NaN, past 2^60).
+// closer to float64 than the float32 chain (the rows where it would not be run
+// in float32).  head_split_pack leaves wp NULL for a weight or bias that cannot
+// be split (infinities, NaN, past 2^60, columns of few terms).
 struct HeadSplit {
   char* wp = nullptr;         // owned by the caller (hipFree)
   const float* ci = nullptr;  // inside wp's allocation

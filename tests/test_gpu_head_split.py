@@ -133,7 +133,7 @@ def test_head_split_distant_winner(gpu, rows):
     n, cols, gaps = 18709, [10, 40, 5000, 18708], [87.5, 88.5, 95.0, 126.0, 200.0, 3000.0]
     rng, w, b = _weights(n, rows)
     w *= 0.1
-    w[:4] = w[:, cols] = 0.0
+    w[:4] = 0.0
     w[range(4), cols] = 1.0             # row q of the weight moves class cols[q] alone
     x = rng.standard_normal((rows, K)).astype(np.float32)
     x[:, :4] = 0.0
@@ -168,3 +168,43 @@ def test_head_split_logits_past_float32(gpu, rows):
     ids = np.ascontiguousarray(pairs[:, 1]).view(np.uint32)
     assert (ids == idx)[gap > 1e-4].all()
     assert (np.abs(pairs[:, 0] - p) <= 1e-5 * p).all()
+
+
+@pytest.mark.parametrize("rows,terms,channel", [(64, 1, 1), (320, 4, 1), (320, 32, 1), (64, 64, 1),
+                                                (320, K, 2.0 ** 23), (40, K, 2.0 ** 23)])
+def test_head_split_rows_it_would_lose_on(gpu, rows, terms, channel):
+    """Rows of few terms, and rows with a channel far past the others whose
+    weight is 0: against float64 no further off than the unsplit kernels', whose
+    logits they then have (the order of the sums apart)."""
+    torch = gpu
+    from qppocr_amd import ops
+    rng, w, b = _weights(18709, 7)
+    x = (rng.standard_normal((rows, K)) * 2 * math.sqrt(K / terms)).astype(np.float32)
+    for r in x:
+        r[rng.permutation(K)[terms:]] = 0.0
+    if channel > 1:
+        x[:, 9], w[9] = 3.0 * channel, 0.0
+    print(f"head split {rows} rows of {terms} terms, channel {channel}", flush=True)
+    sess = _session(rows, w, b)
+    got = sess.run(x.reshape(rows, 1, 1, K))[0].reshape(rows, 2)[:, 0]
+    sess.close()
+    t = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    old = ops.linear_softmax_argmax(t(x), t(w), t(b)).cpu().numpy()[:, 0]
+    p, _, _ = _ref(x, w, b)
+    err = lambda v: np.sqrt((((v - p) / p) ** 2).mean())  # noqa: E731
+    print("relative error, session / float32 chain:", err(got), err(old))
+    assert err(got) <= 1.1 * err(old)
+
+
+def test_head_split_refuses_columns_of_few_terms(gpu):
+    torch = gpu
+    from qppocr_amd import ops
+    rng, w, b = _weights(300, 6)
+    w[95:, 200] = 0.0
+    x = rng.standard_normal((70, K)).astype(np.float32)
+    sess = _session(70, w, b)
+    pairs = sess.run(x.reshape(70, 1, 1, K))[0].reshape(70, 2)
+    sess.close()
+    t = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    old = ops.linear_softmax_argmax(t(x), t(w), t(b)).cpu().numpy()
+    assert (pairs.view(np.uint32) == old.view(np.uint32)).all()
