@@ -1263,10 +1263,12 @@ QPH_API int qph_net_create(qph_ctx* ctx, const qph_net_spec* spec,
       // below the 128x128 size, or with an activation or residual (which the
       // one-wave tiles do not take; at 6800 x 1024 x 256 with GELU
       // linear_nt_kernel takes 46 us, the 32x32 GEMM 80): weight kept
-      // transposed for linear_nt_kernel
+      // transposed for linear_nt_kernel, which stores rows N apart (so not where
+      // the output has a padded pitch)
       const int64_t k = n.ws[0], nn = n.ws[1], rows = numel_of(net, n.in) / k;
       const bool plain = n.act.kind == QPH_ACT_NONE && n.in2 < 0;
-      if (!(plain && gemm_takes_wide(rows, nn, 1)) && linear_nt_eligible(rows, nn, k, k)) {
+      if (!(plain && gemm_takes_wide(rows, nn, 1)) && !net->pitch[(size_t)n.out] &&
+          linear_nt_eligible(rows, nn, k, k)) {
         float* d = nullptr;
         rc = hip_check(hipMalloc((void**)&d, (size_t)(k * nn) * 4), "hipMalloc(transposed weight)");
         if (rc) return bail(rc);

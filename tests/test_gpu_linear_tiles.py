@@ -83,3 +83,33 @@ def test_session_wide_linear_rows(gpu, oracle, rows):
     assert_bitexact(got[0], ref[0], f"probabilities {rows}x{n}")
     assert (np.ascontiguousarray(got[1]).view(np.uint32) ==
             np.ascontiguousarray(ref[1]).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("rows,n,form", [(1280, 9001, "relu"), (1159, 9001, "res"), (1280, 9001, "plain"),
+                                         (1280, 9024, "relu")])
+def test_session_wide_linear_softmax(gpu, oracle, rows, n, form):
+    """A linear of the wide size between an activation or a residual and the
+    softmax that alone reads it: its rows may lie padded, 32 floats apart."""
+    from qppocr_amd import _lib, nets
+    from oracle import nets as onets
+    rng = np.random.default_rng(rows + n)
+    k = 64
+    w = (rng.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32)
+    b = (rng.standard_normal(n) * 0.1).astype(np.float32)
+    g = nets.Graph((rows, 1, 1, k))
+    res = -1
+    if form == "res":
+        w0 = (rng.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32)
+        res = g.linear(0, g.weight(w0), g.weight(b[::-1].copy()), act=_lib.ACT_RELU)
+    y = g.linear(0, g.weight(w), g.weight(b), residual=res,
+                 act=_lib.ACT_RELU if form == "relu" else _lib.ACT_NONE)
+    g.outputs = list(g.softmax_argmax(y, n))
+    x = rng.standard_normal((rows, 1, 1, k)).astype(np.float32)
+    print(f"wide linear + softmax {rows} x {k} x {n} {form}", flush=True)
+    sess = nets.HipSession(g)
+    got = sess.run(x)
+    sess.close()
+    ref = onets.run_graph(g, x)
+    assert_bitexact(got[0], ref[0], f"probabilities {rows}x{n} {form}")
+    assert (np.ascontiguousarray(got[1]).view(np.uint32) ==
+            np.ascontiguousarray(ref[1]).view(np.uint32)).all()
