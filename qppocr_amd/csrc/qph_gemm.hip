@@ -526,10 +526,11 @@ __global__ __launch_bounds__(64) void gemm_pw_group_kernel(PwGroup p) {
 }
 
 // The pointwise kernel takes K a multiple of 16, 16-byte aligned rows of A
-// and offsets within 31 bits, up to 512 output channels (the skinny kernel's
-// 32 x 32 tiles measured slower over that range: 96x1089x128 7.9 against 5.2
-// us, 96x25921x64 25.5 against 17.9, 32 maps of 256x36x256 10.9 against 7.8,
-// 256x10000x256 34.1 against 32.1; past it no net here has a conv).
+// and offsets within 31 bits, up to 512 output channels.  The skinny kernel's
+// 32 x 32 tiles measured slower over that range, convs and plain products alike,
+// pointwise / skinny in us: 96x1089x128 5.2 / 7.9, 96x25921x64 15.4 / 25.5, 32 maps of
+// 256x36x256 7.1 / 9.0; 16x1x64 3.5 / 4.1, 512x36x4096 49 / 76, 256x6400x256 19.1 / 23.9,
+// 192x6400x4096 165 / 165.  (Past 512 no net here has a conv.)
 #define PW_MAX_M 512
 static bool pw_eligible(const GemmArgs& g) {
   return !g.trans_out && g.part == nullptr && g.bias_mode != 2 && g.k % 16 == 0 &&
@@ -637,7 +638,8 @@ static void launch_pw_w(int mbw, const GemmArgs& g, int mgroups, dim3 grid, hipS
   switch (mbw) {
     case 1: launch_pw_m<1, WIDE>(g, mgroups, grid, deep, s); break;
     case 2: launch_pw_m<2, WIDE>(g, mgroups, grid, deep, s); break;
-    default: launch_pw_m<3, WIDE>(g, mgroups, grid, deep, s); break;
+    case 3: launch_pw_m<3, WIDE>(g, mgroups, grid, deep, s); break;
+    default: launch_pw_m<4, WIDE>(g, mgroups, grid, deep, s); break;
   }
 }
 
@@ -645,17 +647,27 @@ static int launch_pw(const GemmArgs& g, hipStream_t s) {
   const int mb = (int)ceil_div(g.m, 16);
   const int64_t pgroups = ceil_div(g.n, 16);
   // Row blocks per wave.  A wave holds few loads in flight, so many short waves
-  // beat fewer long ones until the X slabs they re-read cost more: one block,
-  // two from 16384 waves (from 4096 at K >= 128), three at K >= 256.  In us with
-  // one, two and three blocks: 96x147456x32 41.8, 38.3, 39.4 (six: 53.2);
-  // 96x57600x32 17.7, 18.0, 18.1 (six: 27.0); 96x25921x64 15.4, 16.9, 17.4;
-  // 256x10000x256 27.7, 27.8, 33.2; 96x25600x256 36.7, 31.9, 29.3.
+  // beat fewer long ones until the X slabs they re-read cost more, which comes
+  // earlier the deeper K is: up to four blocks (three where they divide M) with at
+  // most one block in nine past M, if 16384 waves are left (K < 96, and then two
+  // blocks), 3200 (K < 192), 1600 or 850 (K >= 768); where one wave's blocks are all
+  // of M, 3200 are enough.  In us with one, two, three and four blocks, * taken:
+  // 32x102400x32 13.5, 10.0*; 48x102400x64 28.5, 27.5, 23.6*; 96x147456x32 41.8,
+  // 38.3*, 39.4; 96x57600x32 17.7*, 18.0, 18.1; 256x25600x64 24.9*, 26.1, 31.2, 31.4;
+  // 128x6400x128 7.4*, 8.4, 9.4, 10.1; 96x25600x256 36.7, 31.9, 29.3*; 128x25600x512
+  // 85.5, 72.0, 67.8, 61.1*; 192x6400x4096 271, 186, 165*, 152; 256x6400x4096 322, 225,
+  // 264, 187*.  Over 614 shapes (M 16 to 512, N 36 to 102400, K 32 to 4096, batches of 1,
+  // 4 and 32) it is 2% from the best of them.
   auto waves = [&](int c) { return pgroups * (int64_t)ceil_div(mb, c) * g.batch; };
+  const int64_t least = g.k >= 768 ? 850 : g.k >= 192 ? 1600 : g.k >= 96 ? 3200 : 16384;
   int mbw = 1;
-  if (g.k >= 256 && mb % 3 == 0 && waves(3) >= 2048)
-    mbw = 3;
-  else if (waves(2) >= 16384 || (g.k >= 128 && waves(2) >= 4096))
-    mbw = 2;
+  for (int c : {mb % 3 ? 4 : 3, mb % 3 ? 3 : 4, 2}) {
+    if (c > mb || (int)(ceil_div(mb, c) * c - mb) * 8 > mb) continue;
+    if (g.k < 96 && c > 2 && c < mb) continue;
+    if (waves(c) < (c == mb ? std::min<int64_t>(least, 3200) : least)) continue;
+    mbw = c;
+    break;
+  }
   const int mgroups = (int)ceil_div(mb, mbw);
   if (pgroups * mgroups >= (1ll << 31)) return fail(QPH_EUNSUPPORTED, "gemm: grid too large");
   dim3 grid((unsigned)(pgroups * mgroups), 1, (unsigned)g.batch);

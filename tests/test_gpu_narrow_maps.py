@@ -35,6 +35,8 @@ def _conv(gpu, oracle, n, c, h, w, m, k, res):
     (2, 32, 7, 9, 300, True), (1, 32, 151, 151, 151, False),
     (1, 16, 520, 512, 40, False),     # two row blocks a wave, one past M
     (2, 128, 101, 163, 96, True), (1, 256, 129, 129, 96, False),   # two, three
+    (4, 32, 128, 128, 48, True), (4, 16, 120, 113, 20, False),     # all of M in a wave
+    (1, 256, 160, 160, 256, True), (4, 768, 41, 39, 120, False),   # four; three, one past M
     (1, 16, 200, 103, 512, False), (4, 128, 6, 6, 512, True)])
 def test_conv1x1_any_map(gpu, oracle, n, c, h, w, m, res):
     _conv(gpu, oracle, n, c, h, w, m, 1, res)
