@@ -634,7 +634,11 @@ __global__ __launch_bounds__(256) void dwpw_kernel(DwPwK p) {
 //    channel ci, from KH input rows loaded straight into registers.  WIDE
 //    (width % 4 == 0, 16-byte aligned): three aligned 16-byte chunks a row
 //    starting 4 columns left of the first output's window centre, each
-//    wholly inside or outside the image.  Otherwise one word a column.  What is
+//    wholly inside or outside the image.  Otherwise the same loads from the
+//    window's first column, at any 4-byte alignment; the columns past a row's
+//    ends are set to 0 after them.  (By the word, 40 loads a 5x5 task, the lanes
+//    of 16 channels met in the same banks: 128 channels of 16x46 pixels 14.0 us,
+//    7.0 now, dwpw_kernel 8.4; of 64x90 24.9, 10.7 and 21.7.)  What is
 //    outside reads 0 through the buffer range check, which is the zero
 //    padding.  acc = fma(w, x, acc) over ky then kx from 0, + bias,
 //    activation; slots past the row or the image store 0.
@@ -719,31 +723,48 @@ __global__ __launch_bounds__(64 * DWPW_REG_WAVES) void dwpw_reg_kernel(DwPwK p) 
       const int iy0 = oy * p.sh - p.ph;
       const int wx = ox * SW - (WIDE ? 4 : KW / 2);    // window column 0
       float r[KH][4 * NV];
+      // words of the image before column wx of window row ky
+      auto row = [&](int ky) { return ci * (int)plane + (iy0 + ky) * p.w + wx; };
+      auto row_ok = [&](int ky) { return gok && iy0 + ky >= 0 && iy0 + ky < p.h; };
+      // a chunk's first word (!WIDE: kept inside the image)
+      const int last = C * (int)plane - 4;
+      auto at = [&](int ky, int v) {
+        return WIDE ? row(ky) + 4 * v : min(max(row(ky) + 4 * v, 0), last);
+      };
 #pragma unroll
-      for (int ky = 0; ky < KH; ky++) {
-        const int iy = iy0 + ky;
-        const bool rok = gok && iy >= 0 && iy < p.h;
-        const int base = ci * (int)plane + iy * p.w;
-        if constexpr (WIDE) {
+      for (int ky = 0; ky < KH; ky++)
 #pragma unroll
-          for (int v = 0; v < NV; v++) {
-            const int ix = wx + 4 * v;
-            const unsigned off =
-                rok && ix >= 0 && ix < p.w ? (unsigned)((base + ix) * 4) : OOB;
-            const f32x4 q =
-                __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, 0));
+        for (int v = 0; v < NV; v++) {
+          const int ix = wx + 4 * v;
+          const bool ok = row_ok(ky) && (!WIDE || (ix >= 0 && ix < p.w));
+          const f32x4 q = __builtin_bit_cast(
+              f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                         xr, ok ? (unsigned)(at(ky, v) * 4) : OOB, 0, 0));
 #pragma unroll
-            for (int j = 0; j < 4; j++) r[ky][4 * v + j] = q[j];
-          }
-        } else {
+          for (int j = 0; j < 4; j++) r[ky][4 * v + j] = q[j];
+        }
+      if constexpr (!WIDE) {
+        // the image's first and last rows: words of chunks that were moved, back
+        // to their places (what falls outside is past the row's ends)
+        const int top = max(-iy0, 0), bottom = min(KH, p.h - iy0) - 1;
+        if (row(top) < 0 || row(bottom) + 4 * NV > C * (int)plane) {
 #pragma unroll
-          for (int j = 0; j < NC; j++) {
-            const int ix = wx + j;
-            const unsigned off =
-                rok && ix >= 0 && ix < p.w ? (unsigned)((base + ix) * 4) : OOB;
-            r[ky][j] =
-                __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, off, 0, 0));
-          }
+          for (int ky = 0; ky < KH; ky++)
+#pragma unroll
+            for (int v = 0; v < NV; v++) {
+              const int d = at(ky, v) - (row(ky) + 4 * v);
+              float* q = r[ky] + 4 * v;
+              const float q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+#pragma unroll
+              for (int j = 0; j < 4; j++)
+                q[j] = j == d ? q0 : j - 1 == d ? q1 : j - 2 == d ? q2 : q3;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NC; j++) {
+          const bool in = (unsigned)(wx + j) < (unsigned)p.w;
+#pragma unroll
+          for (int ky = 0; ky < KH; ky++) r[ky][j] = in ? r[ky][j] : 0.0f;
         }
       }
       // the channel's taps, four a load (4-byte aligned)

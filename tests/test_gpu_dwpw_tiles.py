@@ -1,6 +1,6 @@
 """Depthwise + pointwise blocks in the register-fed kernel: tiles of 16, 32 and
-64 pixels, rows that are no multiple of four pixels (one-word loads, partial
-groups), single-group rows, slices of M past eight channel blocks, several
+64 pixels, rows that are no multiple of four pixels (unaligned loads, chunks
+past a row's and the image's ends, partial groups), single-group rows, slices of M past eight channel blocks, several
 images, and the channel-last store."""
 import numpy as np
 import pytest
@@ -19,7 +19,11 @@ pytestmark = pytest.mark.gpu
     (1, 128, 128, 96, 96, 5, 1, False), (1, 128, 256, 11, 27, 3, 2, False),
     (1, 128, 130, 4, 1, 3, 1, False), (2, 128, 17, 3, 5, 5, 1, False),
     (1, 32, 48, 1, 2, 3, 1, False), (9, 64, 64, 12, 48, 3, 1, False),
-    (2, 32, 64, 6, 21, 3, 2, True)])
+    (2, 32, 64, 6, 21, 3, 2, True),
+    (1, 16, 16, 1, 1, 5, 1, False), (2, 16, 32, 1, 1, 3, 2, False), (1, 16, 16, 9, 1, 5, 1, False),
+    (3, 16, 16, 2, 3, 5, 1, False), (1, 16, 16, 1, 7, 3, 1, False), (2, 32, 32, 2, 2, 3, 2, False),
+    (1, 64, 64, 17, 18, 5, 1, False), (2, 128, 128, 17, 19, 3, 2, False),
+    (1, 128, 128, 16, 18, 5, 1, False), (2, 16, 16, 31, 405, 3, 2, False)])
 def test_dwpw_tiles(gpu, oracle, n, c, m, h, w, k, s, trans):
     from qppocr_amd import _lib, nets
     from oracle import nets as onets
