@@ -529,7 +529,9 @@ __global__ __launch_bounds__(256) void conv3x3_direct_group_kernel(DirectConvGro
 // 4, so a 16-byte halo group lies wholly inside or wholly outside a row.
 // Other widths (NARROW: the coarse levels of a page whose sides are not
 // multiples of 128) bring the same halo words by 20 one-word loads, 32 loads
-// a chunk in all.
+// a chunk in all.  One such member makes its whole launch NARROW: the two forms
+// side by side, each member its own, took 244.6 us instead of 242.3 on a
+// 736x1280 page and 442.7 instead of 438.8 on 1440x1440 (160x416, 960x1120: equal).
 // Each direct3x3_unit step costs two vector-memory loads per lane; here a
 // step is three LDS reads and two MFMAs.
 
@@ -564,15 +566,6 @@ struct LdsConvGroup {
   int n;
 };
 
-// The ring stages are three __shared__ arrays of their own, picked at compile
-// time (the chunk loop is unrolled over the ring): that is what lets the
-// compiler tell the loads into one stage from the reads of another and place
-// no wait of its own before the operand reads.  The fixed costs around the
-// chunk loop are kept short: the first two chunks' loads go out before
-// anything else is read (bias terms included), a chunk's operands are all
-// read from LDS before its MFMAs (so the reads' latency is paid once a chunk,
-// not once a step), and AK (0 none, 2 ReLU, -1 any kind through act_apply)
-// keeps the epilogue free of the generic activation switch.
 // The conv-transpose pair over NJ tiles of 16 conv outputs of a row, columns
 // pox + 16 j, that this wave wrote to hh ([pixel][CV_HP]): the A operands and
 // w2 through fb, then the products, the second chain and the sigmoid.
@@ -635,6 +628,15 @@ __device__ __forceinline__ void convt_finish(const DirectConvK& p, const ConvtEp
   }
 }
 
+// The ring stages are three __shared__ arrays of their own, picked at compile
+// time (the chunk loop is unrolled over the ring): that is what lets the
+// compiler tell the loads into one stage from the reads of another and place
+// no wait of its own before the operand reads.  The fixed costs around the
+// chunk loop are kept short: the first two chunks' loads go out before
+// anything else is read (bias terms included), a chunk's operands are all
+// read from LDS before its MFMAs (so the reads' latency is paid once a chunk,
+// not once a step), and AK (0 none, 2 ReLU, -1 any kind through act_apply)
+// keeps the epilogue free of the generic activation switch.
 template <int AK, bool ONE, bool CVT = false, bool NARROW = false>
 __device__ __forceinline__ void lds_conv_tile(const DirectConvK& p, int tiles_x, int tile,
                                               float* s0, float* s1, float* s2, float* s3,
@@ -1310,19 +1312,39 @@ static void launch_lds_ring(const LdsConvGroup& g, dim3 grid, bool narrow, hipSt
 }
 
 // Whether the LDS kernel takes the convs of one launch.  With the halo by
-// one-word loads it needs enough tiles to fill the CUs: 96 -> 24 channels,
-// direct against LDS: 80x81 (120 tiles) 11.1 and 13.5 us, 100x101 (200) 15.7
-// and 13.6, 160x161 (480) 25.6 and 21.6; 32 -> 32 channels the same way round.
+// one-word loads its chunks take up to 1.4 times their aligned time, and the direct
+// kernels are the faster where its tiles are few, ragged or half padding.
+// Measured on 1680 convs of 8 to 256 channels and 3000 to 60000 pixels, direct / LDS:
+// - from 160 tiles; up to 16 outputs (half of every step is padding) only with 8
+//   channels and three tiles a CU: 8 -> 16 6.3 / 5.5 us, 32 -> 16 9.0 / 9.9, 96 -> 16
+//   16 / 20;
+// - more outputs: always up to 16 channels (16 -> 24 11.3 / 8.2), up to 32 with 0.6 of
+//   the tiles' pixels in the image, past that (a tile a CU and round takes so long
+//   that the last round shows) with 0.7 of whole rounds' (96 -> 24 of four 64x98 25 / 21,
+//   256 -> 24 200x81, which is 312 tiles, 31 / 45).
+// Of the direct kernels' time 0.94 over all of them, 1.09 at most.
+// A group's direct form runs 16 x 16 units, two waves a SIMD at 2048 (the neck of
+// a 640x288 page, 1915 units: direct 18, LDS 22 us; of 896x224, 2085: 25 and 21).
 #define LDS_NARROW_TILES 160
+#define LDS_NARROW_UNITS 2048
 static bool lds3x3_pays(const ConvArgs* a, int n) {
-  int64_t tiles = 0;
+  int64_t tiles = 0, px = 0, units = 0, m = a[0].m;
   bool narrow = false;
   for (int i = 0; i < n; i++) {
     if (!lds3x3_eligible(a[i])) return false;
     narrow = narrow || !lds3x3_wide(a[i]);
     tiles += (int64_t)ceil_div(a[i].ow, 32) * ceil_div(a[i].oh, 2) * a[i].n;
+    px += a[i].oh * a[i].ow * a[i].n;
+    units += (int64_t)ceil_div(a[i].m, 16) * ceil_div(a[i].oh * a[i].ow, 16) * a[i].n;
+    m = std::min(m, a[i].m);
   }
-  return !narrow || tiles >= LDS_NARROW_TILES;
+  if (!narrow) return true;
+  if (n > 1) return m > 16 && units >= LDS_NARROW_UNITS;
+  if (tiles < LDS_NARROW_TILES) return false;
+  if (m <= 16) return a->c <= 8 && tiles <= 768;
+  if (a->c <= 16) return true;
+  if (a->c <= 32) return 5 * px >= 3 * 64 * tiles;
+  return 10 * px >= 7 * 64 * ((tiles + 255) / 256 * 256);
 }
 
 // Whether the tall kernel takes them (lds3x3_pays already holds): from some two

@@ -45,7 +45,9 @@ def test_conv1x1_any_map(gpu, oracle, n, c, h, w, m, res):
 @pytest.mark.parametrize("n,c,h,w,m,res", [
     (1, 8, 320, 1, 24, False), (1, 24, 161, 33, 32, True), (2, 96, 81, 63, 24, False),
     (5, 32, 64, 31, 5, False), (1, 40, 107, 90, 17, True),
-    (1, 32, 78, 98, 32, False), (1, 32, 80, 98, 32, False)])   # 156 and 160 tiles
+    (1, 32, 78, 98, 32, False), (1, 32, 80, 98, 32, False),    # 156 and 160 tiles
+    (1, 8, 128, 97, 16, True), (1, 24, 120, 94, 32, True), (1, 16, 107, 90, 17, False),
+    (4, 96, 64, 98, 24, False), (1, 40, 270, 95, 20, True), (4, 8, 120, 113, 9, False)])
 def test_conv3x3_any_width(gpu, oracle, n, c, h, w, m, res):
     _conv(gpu, oracle, n, c, h, w, m, 3, res)
 
@@ -57,7 +59,7 @@ def test_conv3x3_tall(gpu, oracle, n, c, h, w, m, res):
     _conv(gpu, oracle, n, c, h, w, m, 3, res)
 
 
-@pytest.mark.parametrize("h,w", [(96, 160), (224, 416), (960, 992)])
+@pytest.mark.parametrize("h,w", [(96, 160), (224, 416), (512, 544), (960, 992)])
 def test_det_net_odd_coarse_levels(gpu, oracle, h, w):
     from qppocr_amd import nets
     from oracle import nets as onets
