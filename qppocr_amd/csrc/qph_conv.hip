@@ -1349,15 +1349,21 @@ static bool lds3x3_pays(const ConvArgs* a, int n) {
 
 // Whether the tall kernel takes them (lds3x3_pays already holds): from some two
 // workgroups a CU on (at 428 tiles, the neck of a 960x544 page, it took 45 us
-// against 41).
+// against 41), unless its last round is so empty that the two-row tiles end
+// first.  A tall round takes 1.5 to 1.6 two-row ones: of four 37x400 maps (520 tiles,
+// three rounds against four) 96 -> 24 35.3 us in two-row tiles and 38.9, 256 -> 24
+// 77.8 and 90.7; in three rounds against five 0.89 of the two-row time over 24
+// shapes, in two against four 0.84, from four on 0.73 to 0.84.
 #define TALL_MIN_TILES 480
 static bool tall3x3_pays(const ConvArgs* a, int n) {
-  int64_t tiles = 0;
+  int64_t tiles = 0, two = 0;
   for (int i = 0; i < n; i++) {
     if (a[i].m <= 16 || a[i].m > LT_WC) return false;
-    tiles += (int64_t)ceil_div(a[i].ow, 32) * ceil_div(a[i].oh, 4) * a[i].n;
+    const int64_t cols = ceil_div(a[i].ow, 32) * a[i].n;
+    tiles += cols * ceil_div(a[i].oh, 4);
+    two += cols * ceil_div(a[i].oh, 2);
   }
-  return tiles >= TALL_MIN_TILES;
+  return tiles >= TALL_MIN_TILES && 8 * ((tiles + 255) / 256) <= 5 * ((two + 255) / 256);
 }
 
 template <int AK>

@@ -54,7 +54,8 @@ def test_conv3x3_any_width(gpu, oracle, n, c, h, w, m, res):
 
 @pytest.mark.parametrize("n,c,h,w,m,res", [
     (1, 8, 481, 97, 24, True), (1, 16, 477, 128, 17, False),   # 484 and 480 tiles
-    (3, 24, 161, 124, 23, False), (1, 40, 479, 100, 20, True), (2, 32, 240, 127, 24, False)])
+    (3, 24, 161, 124, 23, False), (1, 40, 479, 100, 20, True), (2, 32, 240, 127, 24, False),
+    (4, 8, 37, 400, 24, True)])     # 520 tiles, but 988 of two rows
 def test_conv3x3_tall(gpu, oracle, n, c, h, w, m, res):
     _conv(gpu, oracle, n, c, h, w, m, 3, res)
 
