@@ -1570,15 +1570,21 @@ static void launch_lt(const LinArgs& g, hipStream_t s) {
     hipLaunchKernelGGL((linear_nt_kernel<TM, TN, NS, 0>), grid, dim3(256), 0, s, g, ntiles, per_xcd);
 }
 
-// Tile shape and ring depth as measured on the rec linears (1280 to 6800 rows, K
-// 256 / 1024, N 256..1024) and 1x1 convs (K 64..256).  Up to three 32x32
-// tiles per CU, three stages (48 KB, three workgroups per CU): 1280 x 256 x
-// 1024 14.0 us against 15.5 with two stages and 15.5 with 32x64 tiles.  Past
-// that the tiles come in rounds anyway and two stages (32 KB, five
-// workgroups) hide more: 6800 x 256 x 1024 43.0 -> 39.2 us, 6800 x 256 x 256
-// 16.3 -> 14.4.  From N = 512 on such launches take 32x64 tiles (each x slab
-// read for twice the columns): 6800 x 1024 x 256 59.1 -> 45.8, 6800 x 768 x 256
-// 40.6 -> 31.4, 1280 x 1024 x 256 13.5 -> 12.7 (32x32: 47.8, 34.1, 13.4).
+// Tile shape and ring depth, by K, N and the rounds of 32x32 tiles over the CUs,
+// measured on 861 linears (320 to 6800 rows, K 192 to 2048, N 64 to 2000).  In us
+// with three 32x32 stages (48 KB, three workgroups a CU), two (32 KB, five) and
+// 32x64 tiles in two stages, * taken:
+// - up to three rounds three stages: 1280 x 256 x 1024 14.0*, 15.5, 15.5;
+// - K up to 256, more rounds: two stages, from N = 512 on 32x64 tiles (each x slab
+//   read for twice the columns): 6800 x 256 x 256 16.3, 14.4*; 6800 x 1024 x 256
+//   59.1, 47.8, 45.8*; 6800 x 768 x 256 40.6, 34.1, 31.4*;
+// - deeper K: in the fourth round two stages (the fourth workgroup of a CU: 2000 x
+//   512 x 2048 0.78 and 0.90 of three stages' time), in the fifth three (4800 x 256 x
+//   1024 0.87 and 0.94 of the others'); past it two, but three below N = 512 at
+//   K >= 1024 (a rec pass of 40 lines of 1088 pixels, two such linears, 575*, 579, 574;
+//   of 50 688*, 692, 706), and 32x64 from N = 512 in the sixth round (3000 x 512 x
+//   512 0.85, two stages 0.95) and, of rows 4 KB apart, after it (1280 x 2000 x 1024 56, 56, 49*;
+//   x 512 35, 33*, 35).
 // 64-row tiles were never the fastest.
 int launch_linear_nt(const LinArgs& g, hipStream_t s) {
   if (!linear_nt_eligible(g.m, g.n, g.k, g.lda))
@@ -1587,9 +1593,12 @@ int launch_linear_nt(const LinArgs& g, hipStream_t s) {
   QPH_TRY(device_cus(nullptr, &cus_i));
   const int64_t tiles = (int64_t)ceil_div(g.m, 32) * ceil_div(g.n, 32);
   const int64_t cus = cus_i;
-  if (g.k > 128 && tiles <= 3 * cus)
+  const bool deep = g.k > 256, four = tiles <= 4 * cus;
+  if (g.k > 128 && (tiles <= 3 * cus ||
+                    (!four && deep && (tiles <= 5 * cus || (g.k >= 1024 && g.n < 512)))))
     launch_lt<32, 32, 3>(g, s);
-  else if (g.k > 128 && g.n >= 512)
+  else if (g.k > 128 && g.k <= 1024 && g.n >= 512 &&
+           !(deep && (four || (g.k < 1024 && tiles > 6 * cus))))
     launch_lt<32, 64, 2>(g, s);
   else
     launch_lt<32, 32, 2>(g, s);

@@ -15,7 +15,9 @@ pytestmark = pytest.mark.gpu
     (1281, 192, 609, "plain"),      # 41 x 20 tiles of 32 x 32: two stages, 32 x 64
     (777, 256, 1024, "gelu"), (800, 320, 992, "res"), (2600, 192, 511, "plain"),
     (3001, 256, 300, "res"), (6200, 128, 130, "plain"),
-    (9000, 192, 1010, "gelu"), (9000, 256, 1000, "res")])
+    (9000, 192, 1010, "gelu"), (9000, 256, 1000, "res"),
+    (1700, 320, 530, "gelu"), (4300, 320, 250, "res"), (5300, 1024, 250, "plain"),  # rounds 4 to 6
+    (2700, 320, 513, "plain")])
 def test_session_linear_tiles(gpu, oracle, rows, k, n, form):
     from qppocr_amd import _lib, nets
     from oracle import nets as onets
