@@ -907,6 +907,8 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
+        "dtype_detail": "f32 tensors, weights and accumulation; the fused rec head's products run "
+                        "on pairs of float16 terms per f32 operand (three float16 MFMAs a product)",
         "data": "synthetic (seeded inputs, random-init weights)",
         "config": {"workload": "det 1x3x640x640 + rec 32x3x48x320 per step, "
                                "rec ending in the CTC (value, index) pairs",

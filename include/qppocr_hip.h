@@ -374,9 +374,18 @@ typedef struct {
  * are the same bits). */
 #define QPH_NET_SEPARATE_LAUNCHES 1
 /* A linear whose output only the pairs-only softmax argmax right after it
- * reads (the rec head) runs as one GEMM with the softmax argmax in its
- * epilogue; the logits are never stored (qph_linear_softmax_argmax).  Pairs
- * within float rounding of the unfused path, not bit-identical. */
+ * reads (the rec head) runs with the softmax argmax in its epilogue; the
+ * logits are never stored.  Pairs within float rounding of the unfused path,
+ * not bit-identical: with K = 256 inputs each float32 operand is held as two
+ * float16 terms (22 to 24 bits of its row's or column's largest value) and a
+ * product is three float16 MFMAs into a float32 accumulator, whose values are
+ * closer to float64 than a float32 fma chain's (2.5e-6 against 3.6e-6 relative
+ * on the rec net).  Rows where they would not be (fewer than 96 terms past
+ * 2^-20 of the largest, a largest product past 4096, infinities, NaN) run in
+ * float32, and so does the whole head where a column of the weight is such a
+ * row or K is not 256 (then bit for bit qph_linear_softmax_argmax, which is
+ * float32 at every K).  Without the flag the head is the float32 chain of the
+ * reference. */
 #define QPH_NET_FUSED_HEAD 2
 
 typedef struct qph_net qph_net;

@@ -19,7 +19,9 @@ A launch's time is the median over those replays of its kernels' summed
 durations; its work is the sum over the nodes it covers, less the tensors
 passed between them inside it.  Each launch and kernel class is priced
 against both rooflines (fp32 MFMA 157.3 TFLOP/s, HBM 8 TB/s) and its
-fraction is given at the one it comes closer to."""
+fraction is given at the one it comes closer to.  A launch whose float32
+products run as three float16 ones each (head_split kernels) is priced at a
+third of the float16 MFMA peak (2500 TFLOP/s)."""
 import collections
 import csv
 import json
@@ -27,6 +29,7 @@ import statistics
 import sys
 
 PEAK_TFLOPS = 157.3
+PEAK_SPLIT_TFLOPS = 2500.0 / 3      # float32 products as three float16 ones
 PEAK_GBS = 8000.0
 IDLE_NS = 20000
 GAP_NS = 2000
@@ -120,6 +123,11 @@ def internal_mb(cover):
     return mb
 
 
+def peak_tflops(kernels):
+    """The MFMA peak, in float32 FLOP, of a launch's kernels."""
+    return PEAK_SPLIT_TFLOPS if "head_split" in kernels else PEAK_TFLOPS
+
+
 def summarize(name, graph, rows):
     plan, nodes = graph["plan"], graph["nodes"]
     nk = sum(k for _, _, k in plan)
@@ -146,7 +154,7 @@ def summarize(name, graph, rows):
     lines.append("|---:|---|---|---|---:|---:|---:|---:|---:|---:|---|")
     for j, (kn, first, cnt, ops, us, fl, by) in enumerate(launches):
         tf, gb = fl / (us * 1e-6) / 1e12, by / (us * 1e-6) / 1e9
-        fm, fh = tf / PEAK_TFLOPS, gb / PEAK_GBS
+        fm, fh = tf / peak_tflops(kn), gb / PEAK_GBS
         lines.append(f"| {j} | `{kn}` | {first}-{first + cnt - 1} | {ops} | {us:.2f} | "
                      f"{fl / 1e9:.4f} | {by / 1e6:.2f} | {tf:.2f} | {gb:.0f} | {max(fm, fh):.3f} | "
                      f"{'mfma' if fm >= fh else 'hbm'} |")
@@ -164,7 +172,7 @@ def summarize(name, graph, rows):
     for f, (n, us, fl, by) in sorted(fam.items(), key=lambda kv: -kv[1][1]):
         tf, gb = fl / (us * 1e-6) / 1e12, by / (us * 1e-6) / 1e9
         lines.append(f"| `{f}` | {n} | {us:.1f} | {us / total:.2f} | {tf:.2f} | "
-                     f"{tf / PEAK_TFLOPS:.3f} | {gb:.0f} | {gb / PEAK_GBS:.3f} |")
+                     f"{tf / peak_tflops(f):.3f} | {gb:.0f} | {gb / PEAK_GBS:.3f} |")
     lines.append("")
     return lines
 
@@ -180,7 +188,8 @@ def main(argv):
            "of the launch overhead).  Work per launch: the algorithmic flops and bytes of the "
            "nodes it covers (each input, weight and output counted once; a tensor passed between "
            "two nodes inside one launch not at all); frac: against the "
-           "roofline the launch comes closer to (fp32 MFMA 157.3 TFLOP/s, HBM 8 TB/s).", ""]
+           "roofline the launch comes closer to (fp32 MFMA 157.3 TFLOP/s, HBM 8 TB/s; the fused "
+           "head's float32 products run as three float16 ones: a third of 2500 TFLOP/s).", ""]
     for name in ("det", "rec"):
         out += summarize(name, rep[name], rows)
     print("\n".join(out))

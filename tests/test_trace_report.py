@@ -116,3 +116,19 @@ def test_main_writes_both_graphs(tmp_path, capsys):
     out = capsys.readouterr().out
     assert "### det: 2 launches (2 kernels), 4 replays" in out
     assert "### rec: 3 launches (4 kernels), 4 replays" in out
+
+
+def test_split_head_is_priced_at_a_third_of_the_float16_peak(tmp_path):
+    t = Trace()
+    for _ in range(4):
+        t.run(0, ["k_stem", "k_mid", "head_split_kernel", "head_split_pairs_kernel"])
+    trace = tmp_path / "t.csv"
+    with open(trace, "w", newline="") as f:
+        w = csv.DictWriter(f, fieldnames=FIELDS)
+        w.writeheader()
+        w.writerows(t.rows)
+    lines = tr.summarize("rec", nodes_json(), list(csv.DictReader(open(trace))))
+    head = [ln for ln in lines if "head_split_kernel + head_split_pairs_kernel" in ln]
+    # 4 GFLOP in 2 us: 2000 TFLOP/s of float32
+    assert head[0].split("|")[10].strip() == f"{2000 / (2500 / 3):.3f}"
+    assert head[1].split("|")[6].strip() == f"{2000 / (2500 / 3):.3f}"
